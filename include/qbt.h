@@ -246,8 +246,8 @@ int qbt_profile_end(qbt_ctx* ctx, qbt_profile* out);
  * reorder 0) traces its camera and shadow rays in one persistent launch, the
  * shadow rays of finished pixels taken by waves whose camera work has run
  * dry, instead of a camera launch, then a shadow launch: 0 = never, 1 =
- * where it pays (default: two or more lights and 1 to 16 camera rays per lane
- * of the full persistent grid), 2 = always. Results never depend on these. */
+ * where it pays (default: nowhere at present), 2 = always. Results never
+ * depend on these. */
 typedef struct qbt_tuning {
     int path;
     int block_threads;
@@ -257,7 +257,7 @@ typedef struct qbt_tuning {
     int reorder;
     int graph;
     int strip;
-    int merge; /* 1: camera and shadow rays of an exact render in one launch (k_frame) */
+    int merge; /* 2: camera and shadow rays of an exact render in one launch (k_frame) */
 } qbt_tuning;
 
 int qbt_get_tuning(qbt_ctx* ctx, qbt_tuning* out);

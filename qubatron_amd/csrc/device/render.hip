@@ -56,6 +56,7 @@
 #include "pixel.hpp"
 #include "qbt.h"
 #include "qbt_internal.hpp"
+#include "split.hpp"
 #include "trace.hpp"
 
 #pragma clang fp contract(off)
@@ -66,8 +67,6 @@ using namespace qbt;
 
 namespace {
 
-constexpr int kSeg     = 8;  /* work segments per launch (block b starts in segment b % kSeg: one XCD each) */
-constexpr int kCtrPad  = 64; /* uint32 between refill counters: each on its own 256-byte line */
 constexpr int kNL      = QBT_MAX_LIGHTS_RENDER;
 
 /* batch counters (uint32), zeroed before each batch: the number of shaded
@@ -94,39 +93,6 @@ struct PrimOut {
     uint8_t*  flags; /* QBT_PX_LEAF | QBT_PX_SHADED | QBT_PX_DISCARD */
     uint32_t* cand;  /* per work item: batch pixel index if shaded, else ~0 */
     int*      exp;   /* per pixel expansions (counting renders) */
-};
-
-__device__ __forceinline__ uint32_t seg_bound(uint32_t n, int s) { return (uint32_t) (((uint64_t) n * s) / kSeg); }
-
-/* Wave-uniform refill: hands consecutive work items of the wave's current
- * segment to its idle lanes. Returns the item of this lane or UINT32_MAX. */
-struct Refill {
-    int      seg, left;
-    uint32_t n;
-    __device__ Refill(uint32_t total) : seg((int) (blockIdx.x % kSeg)), left(kSeg), n(total) {}
-
-    __device__ __forceinline__ uint32_t fetch(unsigned* ctr, uint64_t idle, int lane)
-    {
-        const uint32_t nidle  = (uint32_t) __popcll(idle);
-        const int      leader = __ffsll((unsigned long long) idle) - 1;
-        const uint32_t lo = seg_bound(n, seg), hi = seg_bound(n, seg + 1);
-        uint32_t       base = 0;
-        if (lane == leader) base = atomicAdd(&ctr[seg * kCtrPad], nidle);
-        /* readlane of a uniform lane: a scalar, so seg and left stay in
-         * scalar registers */
-        base          = __builtin_amdgcn_readlane(base, leader);
-        uint32_t item = UINT32_MAX;
-        if ((idle >> lane) & 1ull) {
-            uint32_t rank = (uint32_t) __popcll(idle & ((1ull << lane) - 1ull));
-            uint64_t it   = (uint64_t) lo + base + rank;
-            if (it < hi) item = (uint32_t) it;
-        }
-        if ((uint64_t) lo + base + nidle >= hi) { /* this segment is done: move on */
-            seg = (seg + 1) % kSeg;
-            left--;
-        }
-        return item;
-    }
 };
 
 /* Lanes with a ray step until it ends; the wave leaves the loop together
@@ -163,20 +129,29 @@ __device__ __forceinline__ Stack lane_stack(uint32_t* lds, uint32_t* gstack, int
     return GSTK ? make_stack_global(gstack, L, DUAL) : make_stack(lds, L, DUAL);
 }
 
+/* the calling wave's 64 words of LDS for drain(), after the stacks */
+template <bool DUAL, bool GSTK>
+__device__ __forceinline__ uint32_t* wave_mail(uint32_t* lds, int L)
+{
+    const uint32_t stack = GSTK ? 0u : blockDim.x * (uint32_t) (L > 0 ? L : 1) * (DUAL ? 3u : 2u);
+    return lds + stack + (threadIdx.x & ~63u);
+}
+
 /* Camera rays of the batch. Work items 0 .. nspr-1 are the sprite traces
  * (view i / nl, light i % nl: the ray from the camera to the light,
  * octree_fsh.c:452-459, one per view and light; result flags to
  * b.sprite), then nitems pixel items. */
 template <bool CMP, bool DUAL, bool GRID, bool COUNT, bool GSTK>
-__global__ void __launch_bounds__(256) k_primary(SceneDev s, BatchDev b, PrimOut o, uint32_t nitems, uint32_t nspr,
+__global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, PrimOut o, uint32_t nitems, uint32_t nspr,
                                                  int nl, int strip, int* __restrict__ sprite, unsigned* __restrict__ q,
-                                                 unsigned refill, uint32_t* gstack,
+                                                 unsigned refill, GridRule rule, uint32_t* gstack,
                                                  unsigned long long* __restrict__ counters)
 {
     extern __shared__ uint32_t lds[];
+    Refill      rf(nspr + nitems, rule.blocks(nspr + nitems));
+    if (blockIdx.x >= rf.grid) return;
     const Stack st   = lane_stack<DUAL, GSTK>(lds, gstack, s.maxlevel);
     const int   lane = threadIdx.x & 63;
-    Refill      rf(nspr + nitems);
     bool        active = false;
     uint32_t    item = 0, gp = 0;
     int         spr  = -1; /* sprite slot of a sprite lane */
@@ -228,15 +203,18 @@ __global__ void __launch_bounds__(256) k_primary(SceneDev s, BatchDev b, PrimOut
         }
     };
 
-    int fin = ST_CONT; /* status of a ray that ended and awaits its outputs */
+    int      fin   = ST_CONT; /* status of a ray that ended and awaits its outputs */
+    uint32_t first = UINT32_MAX;
+    bool     given = rf.share(lane, first); /* few items: each wave its share, no queue */
     for (;;) {
         if (fin != ST_CONT) { /* rays that ended since the last refill point, together */
             finish(fin);
             fin = ST_CONT;
         }
         const uint64_t idle = __ballot(!active);
-        if (rf.left > 0 && (__popcll(idle) >= (int) refill || idle == ~0ull)) {
-            const uint32_t fetched = rf.fetch(&q[Q_PRIM], idle, lane);
+        if (given || (rf.left > 0 && (__popcll(idle) >= (int) refill || idle == ~0ull))) {
+            const uint32_t fetched = given ? first : rf.fetch(&q[Q_PRIM], idle, lane);
+            given                  = false;
             if (fetched != UINT32_MAX && fetched < nspr) {
                 const int      v = (int) (fetched / (uint32_t) nl), l = (int) (fetched % (uint32_t) nl);
                 const ViewDev& V = b.views[v];
@@ -274,6 +252,14 @@ __global__ void __launch_bounds__(256) k_primary(SceneDev s, BatchDev b, PrimOut
                     o.cand[it] = UINT32_MAX; /* padding item of an edge tile */
                 }
             }
+        }
+        if (!COUNT && rf.left <= 0) { /* the queue is dry: the lanes share the rays that are left */
+            drain<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, wave_mail<DUAL, GSTK>(lds, s.maxlevel),
+                                               [&](int stt) {
+                                                   finish(stt);
+                                                   return false;
+                                               });
+            break;
         }
         if (__ballot(active) == 0ull) {
             if (rf.left <= 0) break;
@@ -510,19 +496,20 @@ __global__ void k_oct_scan(const unsigned* __restrict__ cnt, unsigned* __restric
  * (lexp: per light, counting renders), so the frame does not depend on the
  * order in which rays end (the sample collector applies the same rule). */
 template <bool CMP, bool DUAL, bool GRID, bool COUNT, bool GSTK>
-__global__ void __launch_bounds__(256) k_shadow(SceneDev s, LightsDev L, const uint32_t* __restrict__ lists,
+__global__ void __launch_bounds__(256, DUAL ? 5 : 6) k_shadow(SceneDev s, LightsDev L, const uint32_t* __restrict__ lists,
                                                 size_t lstride, const unsigned* __restrict__ counts, int cstride,
                                                 const float4* __restrict__ isp, uint8_t* __restrict__ lstat,
                                                 size_t npix, unsigned* __restrict__ disc, unsigned* __restrict__ q,
-                                                unsigned refill, uint32_t* gstack, int* __restrict__ lexp,
-                                                unsigned long long* __restrict__ counters)
+                                                unsigned refill, GridRule rule, uint32_t* gstack,
+                                                int* __restrict__ lexp, unsigned long long* __restrict__ counters)
 {
     extern __shared__ uint32_t lds[];
-    const Stack st   = lane_stack<DUAL, GSTK>(lds, gstack, s.maxlevel);
-    const int   lane = threadIdx.x & 63;
     uint32_t    total = 0;
     for (int j = 0; j < L.n; j++) total += counts[j * cstride];
-    Refill      rf(total);
+    Refill      rf(total, rule.blocks(total));
+    if (blockIdx.x >= rf.grid) return;
+    const Stack st   = lane_stack<DUAL, GSTK>(lds, gstack, s.maxlevel);
+    const int   lane = threadIdx.x & 63;
     bool        active = false;
     uint32_t    gp     = 0;
     int         lt     = 0; /* the light of this lane's ray */
@@ -547,15 +534,18 @@ __global__ void __launch_bounds__(256) k_shadow(SceneDev s, LightsDev L, const u
         if (COUNT) lexp[(size_t) lt * npix + gp] = (int) t.exps;
     };
 
-    int fin = ST_CONT; /* status of a ray that ended and awaits its outputs */
+    int      fin   = ST_CONT; /* status of a ray that ended and awaits its outputs */
+    uint32_t first = UINT32_MAX;
+    bool     given = rf.share(lane, first); /* as k_primary */
     for (;;) {
         if (fin != ST_CONT) { /* rays that ended since the last refill point, together */
             finish(fin);
             fin = ST_CONT;
         }
         const uint64_t idle = __ballot(!active);
-        if (rf.left > 0 && (__popcll(idle) >= (int) refill || idle == ~0ull)) {
-            const uint32_t k = rf.fetch(&q[Q_SHADOW], idle, lane);
+        if (given || (rf.left > 0 && (__popcll(idle) >= (int) refill || idle == ~0ull))) {
+            const uint32_t k = given ? first : rf.fetch(&q[Q_SHADOW], idle, lane);
+            given            = false;
             if (k != UINT32_MAX) {
                 /* item k -> (light, index in its list); the light's position by
                  * selects (a per-lane index into the lights would go through
@@ -591,6 +581,14 @@ __global__ void __launch_bounds__(256) k_shadow(SceneDev s, LightsDev L, const u
                     else finish(stt);
                 }
             }
+        }
+        if (!COUNT && rf.left <= 0) { /* as k_primary */
+            drain<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, wave_mail<DUAL, GSTK>(lds, s.maxlevel),
+                                               [&](int stt) {
+                                                   finish(stt);
+                                                   return false;
+                                               });
+            break;
         }
         if (__ballot(active) == 0ull) {
             if (rf.left <= 0) break;
@@ -670,7 +668,7 @@ __device__ __forceinline__ int slot_light(uint32_t k, uint32_t nitems, int nl, u
 }
 
 template <bool CMP, bool DUAL, bool GRID, bool COUNT, bool GSTK>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, DUAL ? 4 : 5)
     k_frame(SceneDev s, BatchDev b, PrimOut o, LightsDev L, uint32_t nitems, uint32_t nspr, int strip,
             int* __restrict__ sprite, uint32_t* __restrict__ slots, uint8_t* __restrict__ lstat, size_t npix,
             unsigned* __restrict__ disc, unsigned* __restrict__ q, unsigned refill_p, unsigned refill_s,
@@ -680,7 +678,7 @@ __global__ void __launch_bounds__(256)
     const Stack st   = lane_stack<DUAL, GSTK>(lds, gstack, s.maxlevel);
     const int   lane = threadIdx.x & 63;
     const int   nl   = L.n;
-    Refill      rp(nspr + nitems), rs(nitems * (uint32_t) nl);
+    Refill      rp(nspr + nitems, gridDim.x), rs(nitems * (uint32_t) nl, gridDim.x);
     bool        active = false;
     uint32_t    gp = 0, k = 0, tag = 0;
     Ray         r = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -800,6 +798,19 @@ __global__ void __launch_bounds__(256)
         return sh;
     };
 
+    /* the next light deferred to this lane's pixel; false if it was skipped */
+    auto start_deferred = [&]() -> bool {
+        uint32_t item = k;
+        if (!(tag & kTagFresh)) (void) slot_light(k, nitems, nl, item);
+        const uint32_t pend = (tag & kTagPend) >> 8;
+        const int      l    = __ffs(pend) - 1;
+        tag                 = kTagShadow | (pend & (pend - 1u)) << 8;
+        k                   = (uint32_t) l * nitems + item;
+        uint32_t* w         = slots + 4 * (size_t) k; /* written by this lane */
+        return start_shadow(l, __uint_as_float(slot_load(w + 1)), __uint_as_float(slot_load(w + 2)),
+                            __uint_as_float(slot_load(w + 3)));
+    };
+
     for (;;) {
         bool hit_now = false, ray_now = false, def_now = false; /* this lane's events of this refill point */
         if (fin != ST_CONT) { /* rays that ended since the last refill point, together */
@@ -808,15 +819,7 @@ __global__ void __launch_bounds__(256)
             fin = ST_CONT;
         }
         if (!active && (tag & kTagPend)) { /* the next deferred light of this lane's pixel */
-            uint32_t item = k;
-            if (!(tag & kTagFresh)) (void) slot_light(k, nitems, nl, item);
-            const uint32_t pend = (tag & kTagPend) >> 8;
-            const int      l    = __ffs(pend) - 1;
-            tag                 = kTagShadow | (pend & (pend - 1u)) << 8;
-            k                   = (uint32_t) l * nitems + item;
-            uint32_t* w         = slots + 4 * (size_t) k; /* written by this lane */
-            ray_now = start_shadow(l, __uint_as_float(slot_load(w + 1)), __uint_as_float(slot_load(w + 2)),
-                                   __uint_as_float(slot_load(w + 3)));
+            ray_now = start_deferred();
             def_now = ray_now;
         }
         /* free lanes: no ray, no deferred light, no outputs still to write */
@@ -894,6 +897,22 @@ __global__ void __launch_bounds__(256)
         w_hit += (uint32_t) __popcll(__ballot(hit_now));
         w_ray += (uint32_t) __popcll(__ballot(ray_now));
         w_def += (uint32_t) __popcll(__ballot(def_now));
+        if (!COUNT && rp.left <= 0 && rs.left <= 0 &&
+            __ballot(fin != ST_CONT || (!active && (tag & kTagPend) != 0u)) == 0ull) {
+            /* both queues are dry: the lanes share the rays that are left; the
+             * lights deferred to their pixels follow in another turn */
+            uint32_t hits = 0;
+            drain<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, wave_mail<DUAL, GSTK>(lds, s.maxlevel),
+                                               [&](int stt) {
+                                                   if (tag & kTagShadow) finish_shadow(stt);
+                                                   else hits += finish_camera(stt) ? 1u : 0u;
+                                                   return false;
+                                               });
+            active = false;
+            w_hit += wave_sum(hits);
+            if (__ballot((tag & kTagPend) != 0u) == 0ull) break;
+            continue;
+        }
         if (__ballot(active) == 0ull) {
             if (rp.left <= 0 && rs.left <= 0 && __ballot((tag & kTagPend) != 0u || fin != ST_CONT) == 0ull) break;
             continue;
@@ -1039,52 +1058,31 @@ __global__ void k_fill_u32n(unsigned* p, size_t n, unsigned v)
 
 inline unsigned nblk(size_t n, unsigned bs = 256) { return (unsigned) ((n + bs - 1) / bs); }
 
-/* Blocks of a persistent traversal launch over `items` rays. All the blocks
- * that fit (6 waves per SIMD for the traversal kernels: VGPRs and LDS
- * stacks) when there are at least kFullGridRays rays per lane of that grid;
- * fewer, 4 waves per SIMD, for shorter launches, where the end of a launch
- * (each wave stepping its last few long rays with most lanes idle once the
- * queue runs dry) is a large share: there each wave serves half as many rays
- * again before the queue runs dry. Measured: the 1080p camera launch of the
- * 90M-point scene (5 rays per lane) -2.6% with 4, the one-light shadow launch
- * of the 10M-point scene (1.3 rays per lane) -8%; 3840x2160 frames (20-30
- * rays per lane) and 64-view batches 5-8% slower with 4. */
-constexpr int kSmallGridWavesPerSimd = 4;
-constexpr int kFullGridRays          = 16;
+/* Blocks of a persistent traversal launch over at most `items` rays: all
+ * that are resident (5 or 6 waves per SIMD for the traversal kernels: VGPRs and
+ * LDS stacks), at most one lane per ray, but not fewer than
+ * kSpreadWavesPerSimd waves per SIMD: those then take fewer rays each
+ * (Refill::share), down to one. A wave alone on its SIMD steps at its own
+ * latency, so a second one is nearly free, and the lanes without a ray take
+ * parts of the others' rays (drain). Measured, k_primary and k_shadow of a
+ * 320x240 frame of the 1M-point scene (77k camera rays, 28k shadow rays):
+ * one wave per SIMD 140 + 108 us, two 128 + 95, three 120 + 104, four 129 +
+ * 124. GridRule says how many of the blocks take part. */
+constexpr int kSpreadWavesPerSimd = 2;
+constexpr int kSmallWavesPerSimd  = 4;
 
 template <class K>
-int resident_blocks(K kernel, int bs, size_t lds)
+int persistent_grid(const qbt_ctx* c, K kernel, int bs, size_t lds, size_t items)
 {
     int per = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, bs, lds) != hipSuccess || per <= 0) {
         (void) hipGetLastError();
         per = 1;
     }
-    return per;
-}
-
-/* lanes of the full resident grid of `kernel` */
-template <class K>
-size_t grid_lanes(qbt_ctx* c, K kernel, int bs, size_t lds)
-{
-    return (size_t) resident_blocks(kernel, bs, lds) * (size_t) c->num_cus * (size_t) bs;
-}
-
-/* whether `items` rays fill the full resident grid of `kernel` (at least
- * kFullGridRays per lane) */
-template <class K>
-bool fills_grid(qbt_ctx* c, K kernel, int bs, size_t lds, size_t items)
-{
-    return items >= (size_t) kFullGridRays * grid_lanes(c, kernel, bs, lds);
-}
-
-template <class K>
-int persistent_grid(qbt_ctx* c, K kernel, int bs, size_t lds, size_t items)
-{
-    const int per = resident_blocks(kernel, bs, lds);
-    if (fills_grid(c, kernel, bs, lds, items)) return per * c->num_cus;
-    const int cap = std::max(1, 4 * kSmallGridWavesPerSimd / std::max(1, bs / 64)); /* blocks per CU */
-    return std::min(per, cap) * c->num_cus;
+    const int wpb  = bs / 64;
+    const int one  = (int) nblk(items, (unsigned) bs), few = (int) nblk(items, (unsigned) wpb);
+    const int fill = std::min(few, 4 * kSpreadWavesPerSimd * c->num_cus / wpb);
+    return std::min(per * c->num_cus, std::max(one, fill));
 }
 
 /* the launch configuration a captured graph depends on (kernel arguments) */
@@ -1146,7 +1144,7 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
     if (COUNT && nl > 0 && (rc = c->dev_alloc(c->wb_lexp, (size_t) npix * 4 * nl))) return rc;
 
     const int      bs     = c->block_threads(s.maxlevel, DUAL);
-    const size_t   lds    = GSTK ? 0 : qbt_stack_bytes(s.maxlevel, DUAL, bs);
+    const size_t   lds    = (GSTK ? 0 : qbt_stack_bytes(s.maxlevel, DUAL, bs)) + sizeof(uint32_t) * kMailWords * bs;
     /* refill thresholds: the tuned one for both launches, else the measured
      * defaults (camera rays are shorter, so their refills cost more of a ray) */
     const bool     tuned     = c->tune_refill > 0 && c->tune_refill <= 64;
@@ -1155,24 +1153,21 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
     auto           kp     = k_primary<CMP, DUAL, GRID, COUNT, GSTK>;
     auto           ks     = k_shadow<CMP, DUAL, GRID, COUNT, GSTK>;
     auto           kf     = k_frame<CMP, DUAL, GRID, COUNT, GSTK>;
-    /* exact renders: camera and shadow rays in one launch (k_frame). Tuning
-     * merge 2 always; merge 1 where it was measured to pay: at least two
-     * lights (shadow work enough to fill the end of the camera pass, a few
-     * long rays on mostly idle SIMDs) and a camera pass of 1 to 16 rays per
-     * lane of the full grid (longer passes keep the separate launches at the
-     * full grid; shorter ones are latency-bound either way) */
-    const size_t cam  = (size_t) nitems + nspr;
-    const bool   auto_merge = nl >= 2 && cam >= grid_lanes(c, kp, bs, lds) && !fills_grid(c, kp, bs, lds, cam);
-    const bool merged = (c->tune_merge == 2 || (c->tune_merge == 1 && auto_merge)) && nl > 0 && !surrogate &&
-                        !collect && !reorder;
+    /* Tuning merge 2: camera and shadow rays of an exact render in one launch
+     * (k_frame). It was the faster form of some renders while the end of the
+     * camera launch left the SIMDs to a few long rays; with those rays shared
+     * out (drain) it is not: 90M points, 1920x1080, 2 lights, three views
+     * 2.22 + 4.09 + 3.46 ms against 2.14 + 4.12 + 3.39 for the two launches,
+     * and 12 views with 4 lights of a scene where a fifth of the pixels are
+     * shaded 4.9 against 3.3 ms (a hand-over slot for every pixel and light). */
+    const bool merged = c->tune_merge == 2 && nl > 0 && !surrogate && !collect && !reorder;
     if (merged && (rc = c->dev_alloc(c->wb_slots, (size_t) nitems * 16 * nl))) return rc;
-    /* resident blocks, but no more than one work item per lane: small
-     * batches then start fewer waves (less launch and refill-counter
-     * contention); shadow items are at most one per batch pixel and light */
+    /* shadow items are at most one per batch pixel and light */
     const size_t   np = (size_t) nitems + nspr, ns = (size_t) npix * (nl > 0 ? nl : 1);
-    const int      gp = std::min(persistent_grid(c, kp, bs, lds, np), (int) nblk(np, (unsigned) bs));
-    const int      gs = std::min(persistent_grid(c, ks, bs, lds, ns), (int) nblk(ns, (unsigned) bs));
-    const int      gf = merged ? std::min(persistent_grid(c, kf, bs, lds, np + ns), (int) nblk(np + ns, (unsigned) bs)) : 0;
+    const int      gp = persistent_grid(c, kp, bs, lds, np), gs = persistent_grid(c, ks, bs, lds, ns);
+    const GridRule rule{(uint32_t) (4 * kSpreadWavesPerSimd * c->num_cus * 64 / bs),
+                        (uint32_t) (4 * kSmallWavesPerSimd * c->num_cus * 64 / bs)};
+    const int      gf = merged ? persistent_grid(c, kf, bs, lds, np + ns) : 0;
     const int gmax = std::max(std::max(gp, gs), gf);
     if (GSTK && (rc = c->dev_alloc(c->wb_gstack, qbt_stack_bytes(s.maxlevel, DUAL, gmax * bs)))) return rc;
 
@@ -1214,7 +1209,7 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
         }
         c->prof_mark_begin(QBT_PROF_PRIMARY);
         kp<<<gp, bs, lds, st>>>(s, b, po, nitems, nspr, nl > 0 ? nl : 1, c->tune_strip, (int*) c->sprite.p, q,
-                                refill, gstk, cnt);
+                                refill, rule, gstk, cnt);
         c->prof_mark_end();
         compact(st, PredCand{po.cand, nitems}, nitems, 1, (uint32_t*) c->wb_bcnt.p, q + Q_NSEL, 1, items, 0);
         if (reorder) {
@@ -1238,7 +1233,7 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
             const unsigned* ln  = surrogate ? q + Q_FB : q + Q_NSEL;
             c->prof_mark_begin(QBT_PROF_SHADOW);
             ks<<<gs, bs, lds, st>>>(s, L, li, lst, ln, surrogate ? 1 : 0, po.isp, (uint8_t*) c->wb_lstat.p, npix,
-                                    (unsigned*) c->wb_disc.p, q, refill_sh, gstk, (int*) c->wb_lexp.p, cnt);
+                                    (unsigned*) c->wb_disc.p, q, refill_sh, rule, gstk, (int*) c->wb_lexp.p, cnt);
             c->prof_mark_end();
         }
         if (collect && (err = qbt_collect_batch(c, s, DUAL, L, lists, lstride, q + Q_NSEL, npix))) return err;

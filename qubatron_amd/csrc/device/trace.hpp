@@ -623,6 +623,72 @@ __device__ __forceinline__ int trace_step_c1(const SceneDev& s, const Ray& r, co
     return over ? ST_ABORT : (t.level == s.maxlevel ? ST_HIT : ST_CONT);
 }
 
+/* The backtrack half of trace_step_c1 on its own: leave the current node and
+ * enter the next pending entry of the deepest level below t.level that has
+ * one (t.pend must name one). Used where a ray's pending entries are handed
+ * to another lane (split.hpp). */
+template <int SEM, bool GRID>
+__device__ __forceinline__ int trace_pop_c1(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
+{
+    const int      level = t.level;
+    const uint32_t below = t.pend & ((1u << level) - 1u);
+    const int      lv    = 31 - __clz((int) below);
+    const uint32_t an    = (uint32_t) st.ns[lv * st.stride];
+    const uint32_t pwv   = st.pw[lv * st.stride];
+    const uint32_t w     = ((pwv & 0xFFFFFu) >> 5) | (pwv & 0xFF000000u);
+    st.pw[lv * st.stride] = w;
+    st.ns[lv * st.stride] = (int) (an - (1u << 30));
+    t.pend ^= (1u << lv) & ~(uint32_t) ((int) an >> 31);
+    int j = lv, src = (int) ((w >> 3) & 3u);
+    while (src == 0 && j > 0) {
+        j--;
+        src = (int) ((st.pw[j * st.stride] >> 3) & 3u);
+    }
+    t.entry      = src != 0 ? midplane_cell<SEM, GRID>(s, r, src, j, t.ix, t.iy, t.iz, level - j) : t.start;
+    const int sh = level - lv, o = (int) (w & 7u);
+    t.ns    = (int) ((an & 0x3FFFFFFFu) + (uint32_t) __popc(__builtin_amdgcn_ubfe(w, 24u, (uint32_t) o)));
+    t.ix    = ((t.ix >> sh) << 1) | (o & 1);
+    t.iy    = ((t.iy >> sh) << 1) | ((o >> 1) & 1);
+    t.iz    = ((t.iz >> sh) << 1) | (o >> 2);
+    t.level = lv + 1;
+    return t.level == s.maxlevel ? ST_HIT : ST_CONT;
+}
+
+/* backtrack (octree_fsh.c:368-375) and pop the next pending entry of the
+ * deepest level below t.level that has one; ST_MISS where none has */
+template <bool CMP, bool DUAL, int SEM, bool GRID>
+__device__ __forceinline__ int trace_pop(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
+{
+    if constexpr (CMP && !DUAL) return trace_pop_c1<SEM, GRID>(s, r, st, t);
+    /* the deepest level with a pending entry, from the per-lane mask (bit l
+     * set while level l has one; the levels between have none) */
+    const int      level = t.level;
+    const uint32_t below = t.pend & ((1u << level) - 1u);
+    if (below == 0u) return ST_MISS;
+    const int lv = 31 - __clz((int) below), sh = level - lv;
+    const int ix = t.ix >> sh, iy = t.iy >> sh, iz = t.iz >> sh;
+    uint32_t  w = st.pw[lv * st.stride];
+    int       k = (int) ((w >> 3) & 7u), cnt = (int) (w & 7u);
+    int       e = (int) ((w >> (8 + 5 * k)) & 31u);
+    int       o = e & 7, src = e >> 3;
+    st.pw[lv * st.stride] = (w & ~(7u << 3)) | ((uint32_t) (k + 1) << 3);
+    t.pend &= k + 1 == cnt ? ~(1u << lv) : ~0u;
+    float4 isp;
+    if (src == 0) {
+        isp = entry_of<SEM, GRID>(s, r, st, lv, ix, iy, iz, t.start);
+    } else {
+        isp = midplane_cell<SEM, GRID>(s, r, src, lv, ix, iy, iz, 0);
+    }
+    t.ns    = child_slot<CMP, SEM>(s.stat, st.ns[lv * st.stride], o, lv);
+    t.nd    = DUAL ? child_slot<CMP>(s.dyn, st.nd[lv * st.stride], o, lv) : 0;
+    t.ix    = (ix << 1) | (o & 1);
+    t.iy    = (iy << 1) | ((o >> 1) & 1);
+    t.iz    = (iz << 1) | (o >> 2);
+    t.entry = isp;
+    t.level = lv + 1;
+    return t.level == s.maxlevel ? ST_HIT : ST_CONT;
+}
+
 /*
  * One step: expand the node just entered and descend into its nearest
  * pending child, or backtrack and descend into the next pending child of an
@@ -718,37 +784,7 @@ __device__ __forceinline__ int trace_step(const SceneDev& s, const Ray& r, const
         }
     }
 
-    /* ---- backtrack (octree_fsh.c:368-375) and pop the next pending ---- */
-    /* the deepest level with a pending entry, from the per-lane mask (bit l
-     * set while level l has one; the levels between have none) */
-    const uint32_t below = t.pend & ((1u << level) - 1u);
-    if (below == 0u) return ST_MISS;
-    const int lv = 31 - __clz((int) below), sh = level - lv;
-    const int ix = t.ix >> sh, iy = t.iy >> sh, iz = t.iz >> sh;
-    {
-        uint32_t w = st.pw[lv * st.stride];
-        int      k = (int) ((w >> 3) & 7u), cnt = (int) (w & 7u);
-        {
-            int e   = (int) ((w >> (8 + 5 * k)) & 31u);
-            int o   = e & 7, src = e >> 3;
-            st.pw[lv * st.stride] = (w & ~(7u << 3)) | ((uint32_t) (k + 1) << 3);
-            t.pend &= k + 1 == cnt ? ~(1u << lv) : ~0u;
-            float4 isp;
-            if (src == 0) {
-                isp = entry_of<SEM, GRID>(s, r, st, lv, ix, iy, iz, t.start);
-            } else {
-                isp = midplane_cell<SEM, GRID>(s, r, src, lv, ix, iy, iz, 0);
-            }
-            t.ns = child_slot<CMP, SEM>(s.stat, st.ns[lv * st.stride], o, lv);
-            t.nd = DUAL ? child_slot<CMP>(s.dyn, st.nd[lv * st.stride], o, lv) : 0;
-            t.ix    = (ix << 1) | (o & 1);
-            t.iy    = (iy << 1) | ((o >> 1) & 1);
-            t.iz    = (iz << 1) | (o >> 2);
-            t.entry = isp;
-            t.level = lv + 1;
-            return t.level == s.maxlevel ? ST_HIT : ST_CONT;
-        }
-    }
+    return trace_pop<CMP, DUAL, SEM, GRID>(s, r, st, t);
 }
 
 /*

@@ -22,6 +22,7 @@
 
 #include "qbt.h"
 #include "qbt_internal.hpp"
+#include "split.hpp"
 #include "trace.hpp"
 #include "pixel.hpp"
 
@@ -323,90 +324,153 @@ __global__ void __launch_bounds__(256) k_render(SceneDev s, ViewDev v, const int
     }
 }
 
-/* batched octree_trace_line (SEM: kSemShader, kSemCpu or kSemParticle) */
+/* The rays of a batch launch: work items of a persistent, lane-refilling
+ * launch as the camera rays of a frame (render.hip), the rays left at the
+ * end split over the idle lanes (drain). start(item, r) fills in the ray and
+ * returns false if the item has none; finish(item, r, t, status) writes the
+ * item's outputs. Returns the lane's aborted rays. */
+template <bool CMP, bool DUAL, int SEM, bool GRID, class Start, class Finish>
+__device__ __forceinline__ unsigned trace_batch(const SceneDev& s, uint32_t n, GridRule rule, unsigned* q,
+                                                uint32_t* lds, Start&& start, Finish&& finish)
+{
+    Refill rf(n, rule.blocks(n));
+    if (blockIdx.x >= rf.grid) return 0u;
+    const Stack    st   = make_stack(lds, s.maxlevel, DUAL);
+    const int      lane = threadIdx.x & 63;
+    uint32_t*      mail = lds + blockDim.x * (uint32_t) (s.maxlevel > 0 ? s.maxlevel : 1) * (DUAL ? 3u : 2u) +
+                     (threadIdx.x & ~63u);
+    constexpr int  refill = 16;
+    bool           active = false;
+    uint32_t       item   = 0;
+    Ray            r      = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    TraceState     t;
+    unsigned       n_abort = 0;
+    int            fin     = ST_CONT;
+    uint32_t       first   = UINT32_MAX;
+    bool           given   = rf.share(lane, first);
+    auto           end     = [&](int stt) {
+        n_abort += stt == ST_ABORT ? 1u : 0u;
+        finish(item, r, t, stt);
+    };
+    for (;;) {
+        if (fin != ST_CONT) { /* rays that ended since the last refill point, together */
+            end(fin);
+            fin = ST_CONT;
+        }
+        const uint64_t idle = __ballot(!active);
+        if (given || (rf.left > 0 && (__popcll(idle) >= refill || idle == ~0ull))) {
+            const uint32_t k = given ? first : rf.fetch(q, idle, lane);
+            given            = false;
+            if (k != UINT32_MAX) {
+                item = k;
+                if (start(item, r)) {
+                    const int stt = trace_begin<SEM>(s, r, t);
+                    if (stt == ST_CONT) active = true;
+                    else end(stt);
+                }
+            }
+        }
+        if (rf.left <= 0) {
+            drain<CMP, DUAL, SEM, GRID>(s, r, st, t, active, mail, [&](int stt) {
+                end(stt);
+                return false;
+            });
+            break;
+        }
+        if (active) step_run<CMP, DUAL, SEM, GRID>(s, r, st, t, active, keep_active(rf, refill), fin);
+    }
+    return n_abort;
+}
+
+/* Batched octree_trace_line (SEM: kSemShader, kSemCpu or kSemParticle). 200k
+ * rays (0.5 a lane) of the 10M-point scene: 523 us with one thread per ray
+ * and every wave waiting for its longest, 233 us as work items. */
 template <bool CMP, bool DUAL, int SEM, bool GRID>
 __global__ void __launch_bounds__(256) k_trace_rays(SceneDev s, const float* __restrict__ org,
-                                                     const float* __restrict__ dir, size_t n, int* __restrict__ status,
+                                                     const float* __restrict__ dir, uint32_t n, GridRule rule,
+                                                     unsigned* __restrict__ q, int* __restrict__ status,
                                                      int* __restrict__ model, int* __restrict__ leaf,
                                                      float4* __restrict__ isp, float4* __restrict__ tlf,
                                                      unsigned long long* __restrict__ counters)
 {
     extern __shared__ uint32_t lds[];
-    const Stack st = make_stack(lds, s.maxlevel, DUAL);
-    size_t      i  = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned    ab = 0;
-    if (i < n) {
-        Ray r = {org[3 * i], org[3 * i + 1], org[3 * i + 2], dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]};
-        Hit h;
-        int stt = trace<CMP, DUAL, SEM, GRID>(s, r, st, h);
-        if (stt == ST_ABORT) ab = 1;
-        int    m = -1, lf = -1;
-        float4 ip = make_float4(0.f, 0.f, 0.f, 0.f), tc = ip;
-        if (stt == ST_HIT) {
-            const int L = s.maxlevel;
-            m           = (h.ns == 0 && L > 0) ? 0 : s.stat.model[h.ns];
-            if (SEM == kSemParticle && particle_model_lost(h.ns)) m = 0; /* its slot-8 address */
-            lf          = CMP ? s.stat.ref[h.ns] : h.ns;
-            ip          = h.isp;
-            float x, y, z, w;
-            cube_at<GRID>(s, L, h.ix, h.iy, h.iz, x, y, z, w);
-            tc = make_float4(x, y, z, w);
-        }
-        if (status) status[i] = stt == ST_ABORT ? -2 : stt;
-        if (model) model[i] = m;
-        if (leaf) leaf[i] = lf;
-        if (isp) isp[i] = ip;
-        if (tlf) tlf[i] = tc;
-    }
+    unsigned ab = trace_batch<CMP, DUAL, SEM, GRID>(
+        s, n, rule, q, lds,
+        [&](uint32_t k, Ray& r) {
+            const size_t i = k;
+            r.px = org[3 * i], r.py = org[3 * i + 1], r.pz = org[3 * i + 2];
+            r.dx = dir[3 * i], r.dy = dir[3 * i + 1], r.dz = dir[3 * i + 2];
+            return true;
+        },
+        [&](uint32_t i, const Ray&, const TraceState& t, int stt) {
+            int    m = -1, lf = -1;
+            float4 ip = make_float4(0.f, 0.f, 0.f, 0.f), tc = ip;
+            if (stt == ST_HIT) {
+                const int L = s.maxlevel;
+                m           = (t.ns == 0 && L > 0) ? 0 : s.stat.model[t.ns];
+                if (SEM == kSemParticle && particle_model_lost(t.ns)) m = 0; /* its slot-8 address */
+                lf          = CMP ? s.stat.ref[t.ns] : t.ns;
+                ip          = t.entry;
+                float x, y, z, w;
+                cube_at<GRID>(s, L, t.ix, t.iy, t.iz, x, y, z, w);
+                tc = make_float4(x, y, z, w);
+            }
+            status[i] = stt == ST_ABORT ? -2 : stt;
+            model[i]  = m;
+            leaf[i]   = lf;
+            isp[i]    = ip;
+            tlf[i]    = tc;
+        });
     ab = wave_sum(ab);
     if ((threadIdx.x & 63) == 0 && ab) atomicAdd(&counters[CNT_ABORT], (unsigned long long) ab);
 }
 
 /* The particle shader's main (particle_vsh.c:345-373), one particle per
- * thread: gravity step, a trace of the static tree (direct layout: the
+ * work item: gravity step, a trace of the static tree (direct layout: the
  * shader's slot address is a function of the reference node index) with
  * that shader's semantics, stop at the leaf corner when it is closer than
- * 10 units, else move. pos/spd may alias pos_out/spd_out. */
+ * 10 units, else move. pos/spd may alias pos_out/spd_out (an item reads its
+ * own before it writes them). 4,095 particles (a few thousand are what the
+ * reference keeps): 311 us as one thread each in 64 waves, 104 us as two
+ * rays a wave with the other lanes taking parts of them. */
 template <bool GRID>
-__global__ void __launch_bounds__(256) k_particles(SceneDev s, const float* pos, const float* spd, size_t n,
-                                                   float* pos_out, float* spd_out,
-                                                   unsigned long long* __restrict__ counters)
+__global__ void __launch_bounds__(256) k_particles(SceneDev s, const float* pos, const float* spd, uint32_t n,
+                                                   GridRule rule, unsigned* __restrict__ q, float* pos_out,
+                                                   float* spd_out, unsigned long long* __restrict__ counters)
 {
     extern __shared__ uint32_t lds[];
-    const Stack  st = make_stack(lds, s.maxlevel, false);
-    const size_t i  = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned     ab = 0;
-    if (i < n) {
-        const float p[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-        float       v[3] = {spd[3 * i], spd[3 * i + 1], spd[3 * i + 2]};
-        float       o[3] = {p[0], p[1], p[2]};
-        if (v[0] > -90000.0f) {
-            v[1] -= 0.4f;
-            Ray r = {p[0], p[1], p[2], v[0], v[1], v[2]};
-            Hit h;
-            const int stt  = trace<false, false, kSemParticle, GRID>(s, r, st, h);
-            bool      stop = false;
-            if (stt == ST_ABORT) ab = 1;
-            if (stt == ST_HIT && h.isp.w > 0.0f) {
+    auto write = [&](size_t i, float px, float py, float pz, float vx, float vy, float vz) {
+        pos_out[3 * i] = px, pos_out[3 * i + 1] = py, pos_out[3 * i + 2] = pz;
+        spd_out[3 * i] = vx, spd_out[3 * i + 1] = vy, spd_out[3 * i + 2] = vz;
+    };
+    unsigned ab = trace_batch<false, false, kSemParticle, GRID>(
+        s, n, rule, q, lds,
+        [&](uint32_t k, Ray& r) {
+            const size_t i = k;
+            r.px = pos[3 * i], r.py = pos[3 * i + 1], r.pz = pos[3 * i + 2];
+            r.dx = spd[3 * i], r.dy = spd[3 * i + 1], r.dz = spd[3 * i + 2];
+            if (r.dx > -90000.0f) {
+                r.dy -= 0.4f;
+                return true;
+            }
+            write(i, r.px, r.py, r.pz, r.dx, r.dy, r.dz); /* at rest */
+            return false;
+        },
+        [&](uint32_t i, const Ray& r, const TraceState& t, int stt) {
+            float ox = r.px + r.dx, oy = r.py + r.dy, oz = r.pz + r.dz, vx = r.dx;
+            bool  stop = false;
+            if (stt == ST_HIT && t.entry.w > 0.0f) {
                 float x, y, z, w;
-                cube_at<GRID>(s, s.maxlevel, h.ix, h.iy, h.iz, x, y, z, w);
-                const float dx = x - p[0], dy = y - p[1], dz = z - p[2];
+                cube_at<GRID>(s, s.maxlevel, t.ix, t.iy, t.iz, x, y, z, w);
+                const float dx = x - r.px, dy = y - r.py, dz = z - r.pz;
                 if (sqrtf(dx * dx + dy * dy + dz * dz) < 10.0f) {
-                    o[0] = x, o[1] = y, o[2] = z;
-                    v[0] = -100000.0f;
+                    ox = x, oy = y, oz = z;
                     stop = true;
                 }
             }
-            if (!stop) {
-                o[0] = p[0] + v[0], o[1] = p[1] + v[1], o[2] = p[2] + v[2];
-                if (o[1] < -10.0f) v[0] = -100000.0f;
-            }
-        }
-        for (int a = 0; a < 3; a++) {
-            pos_out[3 * i + a] = o[a];
-            spd_out[3 * i + a] = v[a];
-        }
-    }
+            if (stop || oy < -10.0f) vx = -100000.0f;
+            write(i, ox, oy, oz, vx, r.dy, r.dz);
+        });
     ab = wave_sum(ab);
     if ((threadIdx.x & 63) == 0 && ab) atomicAdd(&counters[CNT_ABORT], (unsigned long long) ab);
 }
@@ -507,6 +571,12 @@ void qbt_ctx::dev_free(DevBuf& b)
 
 static const size_t kStageBytes = 64u << 20;
 
+/* the context's counters: CNT_N x u64, then the work counters of a ray or
+ * particle batch, each on its own 256-byte line */
+constexpr size_t kRayQueue     = 256;
+constexpr size_t kCounterBytes = kRayQueue + sizeof(unsigned) * kSeg * kCtrPad;
+static_assert(sizeof(unsigned long long) * CNT_N <= kRayQueue, "counters before the queue");
+
 extern "C" int qbt_create(const qbt_opts* opts, qbt_ctx** out)
 {
     if (!out) return QBT_EINVAL;
@@ -538,7 +608,7 @@ extern "C" int qbt_create(const qbt_opts* opts, qbt_ctx** out)
         qbt_destroy(c);
         return QBT_EDEVICE;
     }
-    if (c->dev_alloc(c->stage, kStageBytes) || c->dev_alloc(c->counters, sizeof(unsigned long long) * CNT_N) ||
+    if (c->dev_alloc(c->stage, kStageBytes) || c->dev_alloc(c->counters, kCounterBytes) ||
         c->dev_alloc(c->sprite, sizeof(int) * QBT_MAX_LIGHTS_RENDER * QBT_MAX_VIEWS)) {
         qbt_destroy(c);
         return QBT_ENOMEM;
@@ -1628,23 +1698,26 @@ extern "C" int qbt_trace_rays(qbt_ctx* c, const float* origins, const float* dir
     float4* dtlf = (float4*) (base + off_isp + n * 16);
     HIPCHK(hipMemcpyAsync(dorg, origins, n * 12, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(ddir, dirs, n * 12, hipMemcpyHostToDevice, c->stream));
-    k_zero_u64<<<1, 64, 0, c->stream>>>((unsigned long long*) c->counters.p, CNT_N);
+    k_zero_u64<<<1, 256, 0, c->stream>>>((unsigned long long*) c->counters.p, (int) (kCounterBytes / 8));
     HIPCHK(hipEventRecord(c->ev0, c->stream));
-    const int    bs  = c->block_threads(maxlevel, dual);
-    const size_t lds = qbt_stack_bytes(maxlevel, dual, bs);
-    unsigned     nb  = blocks_for(n, bs);
+    const int      bs   = c->block_threads(maxlevel, dual);
+    const size_t   lds  = qbt_stack_bytes(maxlevel, dual, bs) + sizeof(uint32_t) * kMailWords * bs;
+    const GridRule rule = grid_rule(c, bs);
+    unsigned*      q    = (unsigned*) ((char*) c->counters.p + kRayQueue);
     unsigned long long* cnt = (unsigned long long*) c->counters.p;
     c->prof_mark_begin(QBT_PROF_PRIMARY);
     /* (DUAL, SEM) in {(0,shader), (1,shader), (0,cpu)}: the CPU twin walks the
      * static tree only; the particle copy: static tree, direct layout */
     if (semantics == 2) {
         auto k = grid ? k_trace_rays<false, false, kSemParticle, true> : k_trace_rays<false, false, kSemParticle, false>;
-        k<<<nb, bs, lds, c->stream>>>(s, dorg, ddir, n, dst, dmod, dlf, disp, dtlf, cnt);
+        k<<<persistent_grid(c, k, bs, lds, n), bs, lds, c->stream>>>(s, dorg, ddir, (uint32_t) n, rule, q, dst, dmod,
+                                                                    dlf, disp, dtlf, cnt);
     } else {
         qbt_dispatch4(cmp, dual, semantics == 1, grid, [&](auto C_, auto D_, auto P_, auto G_) {
             constexpr bool kD = decltype(D_)::value && !decltype(P_)::value;
-            k_trace_rays<decltype(C_)::value, kD, decltype(P_)::value ? kSemCpu : kSemShader, decltype(G_)::value>
-                <<<nb, bs, lds, c->stream>>>(s, dorg, ddir, n, dst, dmod, dlf, disp, dtlf, cnt);
+            auto k = k_trace_rays<decltype(C_)::value, kD, decltype(P_)::value ? kSemCpu : kSemShader, decltype(G_)::value>;
+            k<<<persistent_grid(c, k, bs, lds, n), bs, lds, c->stream>>>(s, dorg, ddir, (uint32_t) n, rule, q, dst,
+                                                                        dmod, dlf, disp, dtlf, cnt);
             return 0;
         });
     }
@@ -1688,15 +1761,16 @@ extern "C" int qbt_particle_update(qbt_ctx* c, const float* pos, const float* sp
     float* dspd = dpos + 3 * n;
     HIPCHK(hipMemcpyAsync(dpos, pos, n * 12, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(dspd, spd, n * 12, hipMemcpyHostToDevice, c->stream));
-    k_zero_u64<<<1, 64, 0, c->stream>>>((unsigned long long*) c->counters.p, CNT_N);
+    k_zero_u64<<<1, 256, 0, c->stream>>>((unsigned long long*) c->counters.p, (int) (kCounterBytes / 8));
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     const int    bs  = c->block_threads(maxlevel, false);
-    const size_t lds = qbt_stack_bytes(maxlevel, false, bs);
-    const unsigned nb = blocks_for(n, bs);
+    const size_t lds = qbt_stack_bytes(maxlevel, false, bs) + sizeof(uint32_t) * kMailWords * bs;
+    unsigned*    q   = (unsigned*) ((char*) c->counters.p + kRayQueue);
     unsigned long long* cnt = (unsigned long long*) c->counters.p;
     c->prof_mark_begin(QBT_PROF_PRIMARY);
-    if (grid) k_particles<true><<<nb, bs, lds, c->stream>>>(s, dpos, dspd, n, dpos, dspd, cnt);
-    else k_particles<false><<<nb, bs, lds, c->stream>>>(s, dpos, dspd, n, dpos, dspd, cnt);
+    auto k = grid ? k_particles<true> : k_particles<false>;
+    k<<<persistent_grid(c, k, bs, lds, n), bs, lds, c->stream>>>(s, dpos, dspd, (uint32_t) n, grid_rule(c, bs), q, dpos,
+                                                                dspd, cnt);
     HIPCHK(hipGetLastError());
     c->prof_mark_end();
     HIPCHK(hipEventRecord(c->ev1, c->stream));

@@ -95,33 +95,6 @@ struct PrimOut {
     int*      exp;   /* per pixel expansions (counting renders) */
 };
 
-/* Lanes with a ray step until it ends; the wave leaves the loop together
- * once fewer than `keep` lanes are left (wave-uniform), so that the refill
- * test, the ballots and the merge of the ray state run once per refill,
- * not once per step. A lane whose ray ends keeps its status in `fin` and
- * its state as it is: the caller writes the results of all such lanes
- * together at the next refill point (a lane that ends would otherwise run
- * the output code with one or two lanes of its wave, in most steps). */
-__device__ __forceinline__ int keep_active(const Refill& rf, unsigned refill)
-{
-    return rf.left > 0 ? 65 - (int) refill : 1; /* refill when idle lanes >= refill */
-}
-
-template <bool CMP, bool DUAL, bool GRID>
-__device__ __forceinline__ void step_run(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t, bool& active,
-                                         int keep, int& fin)
-{
-    for (;;) {
-        const int stt = trace_step<CMP, DUAL, false, GRID>(s, r, st, t);
-        if (stt != ST_CONT) {
-            fin    = stt;
-            active = false;
-            break;
-        }
-        if (__popcll(__ballot(1)) < keep) break;
-    }
-}
-
 /* the calling lane's traversal stack: LDS, or global memory (GSTK) */
 template <bool DUAL, bool GSTK>
 __device__ __forceinline__ Stack lane_stack(uint32_t* lds, uint32_t* gstack, int L)
@@ -265,7 +238,7 @@ __global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, Prim
             if (rf.left <= 0) break;
             continue;
         }
-        if (active) step_run<CMP, DUAL, GRID>(s, r, st, t, active, keep_active(rf, refill), fin);
+        if (active) step_run<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, keep_active(rf, refill), fin);
     }
     n_hit   = wave_sum(n_hit);
     n_abort = wave_sum(n_abort);
@@ -594,7 +567,7 @@ __global__ void __launch_bounds__(256, DUAL ? 5 : 6) k_shadow(SceneDev s, Lights
             if (rf.left <= 0) break;
             continue;
         }
-        if (active) step_run<CMP, DUAL, GRID>(s, r, st, t, active, keep_active(rf, refill), fin);
+        if (active) step_run<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, keep_active(rf, refill), fin);
     }
     n_ray   = wave_sum(n_ray);
     n_abort = wave_sum(n_abort);
@@ -924,7 +897,7 @@ __global__ void __launch_bounds__(256, DUAL ? 4 : 5)
                          : rp.left > 0                    ? 65 - (int) refill_p
                          : rs.left > 0                    ? 65 - (int) refill_s
                                                           : 1;
-        if (active) step_run<CMP, DUAL, GRID>(s, r, st, t, active, keep, fin);
+        if (active) step_run<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, keep, fin);
     }
     if (COUNT) n_exp = wave_sum(n_exp);
     if (lane == 0) {
@@ -1058,33 +1031,6 @@ __global__ void k_fill_u32n(unsigned* p, size_t n, unsigned v)
 
 inline unsigned nblk(size_t n, unsigned bs = 256) { return (unsigned) ((n + bs - 1) / bs); }
 
-/* Blocks of a persistent traversal launch over at most `items` rays: all
- * that are resident (5 or 6 waves per SIMD for the traversal kernels: VGPRs and
- * LDS stacks), at most one lane per ray, but not fewer than
- * kSpreadWavesPerSimd waves per SIMD: those then take fewer rays each
- * (Refill::share), down to one. A wave alone on its SIMD steps at its own
- * latency, so a second one is nearly free, and the lanes without a ray take
- * parts of the others' rays (drain). Measured, k_primary and k_shadow of a
- * 320x240 frame of the 1M-point scene (77k camera rays, 28k shadow rays):
- * one wave per SIMD 140 + 108 us, two 128 + 95, three 120 + 104, four 129 +
- * 124. GridRule says how many of the blocks take part. */
-constexpr int kSpreadWavesPerSimd = 2;
-constexpr int kSmallWavesPerSimd  = 4;
-
-template <class K>
-int persistent_grid(const qbt_ctx* c, K kernel, int bs, size_t lds, size_t items)
-{
-    int per = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, bs, lds) != hipSuccess || per <= 0) {
-        (void) hipGetLastError();
-        per = 1;
-    }
-    const int wpb  = bs / 64;
-    const int one  = (int) nblk(items, (unsigned) bs), few = (int) nblk(items, (unsigned) wpb);
-    const int fill = std::min(few, 4 * kSpreadWavesPerSimd * c->num_cus / wpb);
-    return std::min(per * c->num_cus, std::max(one, fill));
-}
-
 /* the launch configuration a captured graph depends on (kernel arguments) */
 struct GraphKey {
     SceneDev s;
@@ -1165,8 +1111,7 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
     /* shadow items are at most one per batch pixel and light */
     const size_t   np = (size_t) nitems + nspr, ns = (size_t) npix * (nl > 0 ? nl : 1);
     const int      gp = persistent_grid(c, kp, bs, lds, np), gs = persistent_grid(c, ks, bs, lds, ns);
-    const GridRule rule{(uint32_t) (4 * kSpreadWavesPerSimd * c->num_cus * 64 / bs),
-                        (uint32_t) (4 * kSmallWavesPerSimd * c->num_cus * 64 / bs)};
+    const GridRule rule = grid_rule(c, bs);
     const int      gf = merged ? persistent_grid(c, kf, bs, lds, np + ns) : 0;
     const int gmax = std::max(std::max(gp, gs), gf);
     if (GSTK && (rc = c->dev_alloc(c->wb_gstack, qbt_stack_bytes(s.maxlevel, DUAL, gmax * bs)))) return rc;

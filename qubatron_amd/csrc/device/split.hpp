@@ -41,6 +41,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
+#ifndef QBT_HOST_BUILD
+#include "qbt_internal.hpp"
+#endif
 #include "trace.hpp"
 
 #pragma clang fp contract(off)
@@ -259,6 +264,66 @@ struct Refill {
         return item;
     }
 };
+
+/* Lanes with a ray step until it ends; the wave leaves the loop together
+ * once fewer than `keep` lanes are left (wave-uniform), so that the refill
+ * test, the ballots and the merge of the ray state run once per refill,
+ * not once per step. A lane whose ray ends keeps its status in `fin` and
+ * its state as it is: the caller writes the results of all such lanes
+ * together at the next refill point (a lane that ends would otherwise run
+ * the output code with one or two lanes of its wave, in most steps). */
+__device__ __forceinline__ int keep_active(const Refill& rf, unsigned refill)
+{
+    return rf.left > 0 ? 65 - (int) refill : 1; /* refill when idle lanes >= refill */
+}
+
+template <bool CMP, bool DUAL, int SEM, bool GRID>
+__device__ __forceinline__ void step_run(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t, bool& active,
+                                         int keep, int& fin)
+{
+    for (;;) {
+        const int stt = trace_step<CMP, DUAL, SEM, GRID>(s, r, st, t);
+        if (stt != ST_CONT) {
+            fin    = stt;
+            active = false;
+            break;
+        }
+        if (__popcll(__ballot(1)) < keep) break;
+    }
+}
+
+/* Blocks of a persistent traversal launch over at most `items` rays: all
+ * that are resident (5 or 6 waves per SIMD for the traversal kernels: VGPRs and
+ * LDS stacks), at most one lane per ray, but not fewer than
+ * kSpreadWavesPerSimd waves per SIMD: those then take fewer rays each
+ * (Refill::share), down to one. A wave alone on its SIMD steps at its own
+ * latency, so a second one is nearly free, and the lanes without a ray take
+ * parts of the others' rays (drain). Measured, k_primary and k_shadow of a
+ * 320x240 frame of the 1M-point scene (77k camera rays, 28k shadow rays):
+ * one wave per SIMD 140 + 108 us, two 128 + 95, three 120 + 104, four 129 +
+ * 124. GridRule says how many of the blocks take part. */
+constexpr int kSpreadWavesPerSimd = 2;
+constexpr int kSmallWavesPerSimd  = 4;
+
+template <class K>
+inline int persistent_grid(const qbt_ctx* c, K kernel, int bs, size_t lds, size_t items)
+{
+    int per = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, bs, lds) != hipSuccess || per <= 0) {
+        (void) hipGetLastError();
+        per = 1;
+    }
+    const int wpb  = bs / 64;
+    const int one  = (int) ((items + bs - 1) / bs), few = (int) ((items + wpb - 1) / wpb);
+    const int fill = std::min(few, 4 * kSpreadWavesPerSimd * c->num_cus / wpb);
+    return std::min(per * c->num_cus, std::max(one, fill));
+}
+
+inline GridRule grid_rule(const qbt_ctx* c, int bs)
+{
+    return {(uint32_t) (4 * kSpreadWavesPerSimd * c->num_cus * 64 / bs),
+            (uint32_t) (4 * kSmallWavesPerSimd * c->num_cus * 64 / bs)};
+}
 
 #endif
 

@@ -3,12 +3,12 @@
  * counterpart: the reference traces every shadow ray,
  * src/qubatron/shaders/octree_fsh.c:426-434).
  *
- *   training   feature kernel -> one fused kernel per minibatch: forward
- *              (bias + ReLU + bf16 between layers), loss and output
- *              gradient, backward through the masked transposed weights and
- *              the weight and bias gradients, 64 samples per wave on the
- *              matrix cores -> sum of the per-block partial gradients ->
- *              Adam on fp32 master weights -> bf16 repack
+ *   training   two kernels per minibatch: features, forward (bias + ReLU +
+ *              bf16 between layers), loss and output gradient, backward
+ *              through the masked transposed weights and the weight and bias
+ *              gradients, 64 samples per block on the matrix cores -> sum of
+ *              the per-block partial gradients, Adam on fp32 master weights,
+ *              bf16 repack
  *   inference  one fused kernel: weights in LDS, 16 queries per wave, the
  *              four layers chained in registers (mlp.hpp)
  *   render     the decision pass of QBT_RENDER_SURROGATE: predicted bits
@@ -21,6 +21,7 @@
  */
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <math.h>
 
@@ -47,13 +48,17 @@ struct RawSample {
 };
 static_assert(sizeof(RawSample) == 40, "sample record");
 
-/* fp32 gradient layout: packed weight matrices (as kP*), then the biases */
-constexpr int kGB1 = kPackN, kGB2 = kGB1 + 64, kGB3 = kGB2 + 64, kGB4 = kGB3 + 64, kGradN = kGB4 + 1;
+/* a block's partial gradients (fp32): the 16 x 16 tiles of dW1, dW2, dW3 as
+ * matrix-core fragments (element 256 t + 4 lane + e), dW4, the biases */
+constexpr int kG2 = 12 * 256, kG3 = kG2 + 16 * 256, kG4 = kG3 + 16 * 256, kGB1 = kG4 + 64, kGB2 = kGB1 + 64,
+              kGB3 = kGB2 + 64, kGB4 = kGB3 + 64, kGradN = kGB4 + 64; /* padded to 64 */
+/* packed weights of the training kernel, after the inference kernels' (kP*): W2 and W3 transposed */
+constexpr int kPT2 = kPackN, kPT3 = kPT2 + 64 * 64, kPackAll = kPT3 + 64 * 64;
 /* biases in LDS for the fused kernels */
 constexpr int kLB1 = 0, kLB2 = 64, kLB3 = 128, kLB4 = 192, kLBN = 196;
 
 struct MlpState {
-    DevBuf   params, m, v, grads, packed, ctr; /* ctr: collected, lit (u64) */
+    DevBuf   params, m, v, packed, ctr; /* ctr: collected, lit (u64) */
     DevBuf   samples, perm, keys, vals, sort_tmp;
     DevBuf   X, gpart, lossbuf, io_x, io_p, io_y, io_a, io_c, flat; /* gpart: k_mlp_train's partial gradients */
     size_t   cap = 0;
@@ -101,12 +106,17 @@ __global__ void k_mlp_init(float* P, uint64_t seed)
     P[i]    = a > 0.0f ? (2.0f * u - 1.0f) * a : 0.0f;
 }
 
-/* fp32 parameters -> padded bf16 weight matrices */
+/* fp32 parameters -> padded bf16 weight matrices, W2 and W3 also transposed */
 __global__ void k_mlp_pack(const float* __restrict__ P, uint16_t* __restrict__ W)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= kPackN) return;
+    if (i >= kPackAll) return;
     float v = 0.0f;
+    if (i >= kPackN) {
+        const int k = (i - kPackN) % (64 * 64), o = k % 64, c = k / 64;
+        W[i]        = f2bf(P[(i < kPT3 ? kW2 : kW3) + o * 64 + c]);
+        return;
+    }
     if (i < kP2) {
         int o = i / 48, c = i % 48;
         v     = c < kMlpIn ? P[kW1 + o * kMlpIn + c] : 0.0f;
@@ -125,61 +135,11 @@ __global__ void k_mlp_pack(const float* __restrict__ P, uint16_t* __restrict__ W
 /* fused training forward and backward                                      */
 /* ------------------------------------------------------------------------ */
 
-constexpr int kChunk = 64; /* samples per chunk: four fragment groups of 16, one per wave */
+constexpr int kChunk = 64; /* samples per chunk: four fragment groups of 16 */
+constexpr int kRow   = 68; /* elements of a row of 64 in LDS (padded: rows start 2 banks apart) */
 
-/* one chunk's activations and gradients, [feature][kChunk] bf16 */
-struct TrainLds {
-    uint16_t x[kMlpInPad * kChunk];
-    uint16_t h1[64 * kChunk], h2[64 * kChunk], h3[64 * kChunk];
-    uint16_t d1[64 * kChunk], d2[64 * kChunk], d3[64 * kChunk], d4[16 * kChunk];
-    float    bias[kLBN];
-};
-
-/* A fragment of W (row-major, `in` columns): rows 16 mt.., columns 16 kb.. */
-__device__ __forceinline__ bf16x4 wfrag(const uint16_t* __restrict__ W, int in, int mt, int kb, int r, int g)
-{
-    return *reinterpret_cast<const bf16x4*>(W + (16 * mt + r) * in + 16 * kb + 4 * g);
-}
-
-/* A fragment of W^T: element (i, k) = W[16 kb + k][16 mt + i] */
-__device__ __forceinline__ bf16x4 wtfrag(const uint16_t* __restrict__ W, int in, int mt, int kb, int r, int g)
-{
-    bf16x4 v;
-    for (int e = 0; e < 4; e++) v[e] = (short) W[(16 * kb + 4 * g + e) * in + 16 * mt + r];
-    return v;
-}
-
-/* D fragment (features 16 t + 4 g + e of sample r) of group j into a
- * [feature][kChunk] LDS array */
-__device__ __forceinline__ void put_frag(uint16_t* __restrict__ a, int t, int j, bf16x4 v, int r, int g)
-{
-    for (int e = 0; e < 4; e++) a[(16 * t + 4 * g + e) * kChunk + 16 * j + r] = (uint16_t) v[e];
-}
-
-/* one 16 x 16 tile of D = A B^T over the chunk's 64 samples (K): A rows
- * 16 mt.. of a, B rows 16 nt.. of b, both [row][kChunk] in LDS */
-__device__ __forceinline__ f32x4 chunk_tile(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, int mt,
-                                            int nt, int r, int g)
-{
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int j = 0; j < kChunk / 16; j++) {
-        const bf16x4 av = *reinterpret_cast<const bf16x4*>(a + (16 * mt + r) * kChunk + 16 * j + 4 * g);
-        const bf16x4 bv = *reinterpret_cast<const bf16x4*>(b + (16 * nt + r) * kChunk + 16 * j + 4 * g);
-        acc             = mfma16(av, bv, acc);
-    }
-    return acc;
-}
-
-/* the gradient tile (rows 16 mt + 4 g + e, column 16 nt + r of a matrix
- * with `in` columns at offset off) into the block's row of partial sums */
-__device__ __forceinline__ void add_tile(float* __restrict__ gp, bool first, int off, int in, int mt, int nt, f32x4 v,
-                                         int r, int g)
-{
-    for (int e = 0; e < 4; e++) {
-        float* q = gp + off + (16 * mt + 4 * g + e) * in + 16 * nt + r;
-        *q       = first ? v[e] : *q + v[e];
-    }
-}
+__device__ __forceinline__ bf16x4 lds4(const uint16_t* a) { return *reinterpret_cast<const bf16x4*>(a); }
+__device__ __forceinline__ void   lds4(uint16_t* a, bf16x4 v) { *reinterpret_cast<bf16x4*>(a) = v; }
 
 __device__ __forceinline__ bf16x4 relu_pack(f32x4 acc, const float* __restrict__ b)
 {
@@ -194,194 +154,247 @@ __device__ __forceinline__ bf16x4 mask_pack(f32x4 acc, bf16x4 h)
                  h[3] > 0 ? acc[3] : 0.0f);
 }
 
-/* the weights as matrix-core A fragments, forward (W) and backward (W^T),
- * held in registers for a whole launch */
-struct TrainFrags {
-    bf16x4 w1[4][3], w2[4][4], w3[4][4], w4[4]; /* W:   rows 16 mt.., columns 16 kb.. */
-    bf16x4 t2[4][4], t3[4][4], t4[4];           /* W^T: rows 16 mt.., columns 16 kb.. */
+/* samples of a minibatch: the store's records perm[off ..] (S not null), or
+ * the feature matrix X[48][B] with labels Y */
+struct TrainBatch {
+    const RawSample* S;
+    const uint32_t*  perm;
+    size_t           off;
+    float            bx, by, bz, bw;
+    const uint16_t*  X;
+    const float*     Y;
+    int              B, n; /* columns, of which valid */
 };
 
-__device__ __forceinline__ void load_train_frags(const uint16_t* __restrict__ W, int r, int g, TrainFrags& F)
-{
-    for (int mt = 0; mt < 4; mt++) {
-        for (int kb = 0; kb < 3; kb++) F.w1[mt][kb] = wfrag(W + kP1, 48, mt, kb, r, g);
-        for (int kb = 0; kb < 4; kb++) {
-            F.w2[mt][kb] = wfrag(W + kP2, 64, mt, kb, r, g);
-            F.w3[mt][kb] = wfrag(W + kP3, 64, mt, kb, r, g);
-            F.t2[mt][kb] = wtfrag(W + kP2, 64, mt, kb, r, g);
-            F.t3[mt][kb] = wtfrag(W + kP3, 64, mt, kb, r, g);
-        }
-        F.w4[mt] = wfrag(W + kP4, 64, 0, mt, r, g);  /* the output row block, K block mt */
-        F.t4[mt] = wtfrag(W + kP4, 64, mt, 0, r, g); /* W4^T rows 16 mt.., its 16 columns */
-    }
-}
-
-/* Forward and backward of the B columns of X (n valid; labels Y), four
- * waves per block. Block b takes the 64-sample chunks b, b + gridDim.x, ...;
- * per chunk wave w runs fragment group w (16 samples) through the four
- * layers as matrix-core fragments (bias, ReLU and bf16 rounding between
- * layers, the rounding points of the oracle), the loss and output gradient
- * (bf16((p - y) / n)), and the backward pass through the transposed weights
- * masked by the ReLU outputs, writing every activation and gradient to LDS;
- * then the four waves share the chunk's 48 weight-gradient tiles (16 x 16,
- * the 64 samples as K) and the bias row sums, added to the block's own row
- * of gp (kGradN floats, no atomics; k_grad_rows sums the rows). The summed
- * BCE goes to *loss. */
+/* Forward and backward of a minibatch, four waves per block; block b takes
+ * the 64-sample chunks b, b + gridDim.x, ... Wave w computes output features
+ * 16 w .. 16 w + 15 of every layer for the chunk's four groups of 16 samples
+ * (its rows of W and W^T are 24 fragments, held in registers), and the same
+ * rows of the weight gradients, whose fragments stay in registers over the
+ * chunks. Rounding points as the oracle's: bias, ReLU and bf16 between
+ * layers, output gradient bf16((p - y) / n). Activations and gradients pass
+ * between the waves through LDS twice: a sample per row (B fragments of the
+ * next layer; two buffers in turn) and a feature per row (both operands of a
+ * weight gradient, the samples as K). The block's gradients go to its row of
+ * gp (no atomics; k_mlp_step sums the rows). loss: the summed BCE is added,
+ * if not null (a training run needs that of its last step only: the double
+ * logarithms are a tenth of the kernel).
+ *
+ * What bounds it: latency, 64 blocks at batch 4096, nine barriers. 12.6 us
+ * a step's launch, features included, against 28 + 8 + 4 us (features, loss
+ * reset) with every wave taking 16 samples through all features: that loaded
+ * 84 weight fragments per wave, two bytes at a time for the transposed ones,
+ * and summed the biases from LDS with all lanes on one bank. */
+template <bool STORE>
 __global__ void __launch_bounds__(256) k_mlp_train(const uint16_t* __restrict__ W, const float* __restrict__ P,
-                                                   const uint16_t* __restrict__ X, const float* __restrict__ Y, int B,
-                                                   int n, float* __restrict__ gp, double* __restrict__ loss)
+                                                   TrainBatch T, float* __restrict__ gp, double* __restrict__ loss)
 {
-    __shared__ TrainLds L;
-    const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
-    for (int i = tid; i < kLBN; i += blockDim.x) {
-        float b = 0.0f;
-        if (i < 64) b = P[kB1 + i];
-        else if (i < 128) b = P[kB2 + i - 64];
-        else if (i < 192) b = P[kB3 + i - 128];
-        else if (i == kLB4) b = P[kB4];
-        L.bias[i] = b;
+    __shared__ __align__(16) uint16_t S0[kChunk * kRow], S1[kChunk * kRow]; /* [sample][feature], in turn */
+    __shared__ __align__(16) uint16_t Xf[kMlpInPad * kRow], H1[64 * kRow], H2[64 * kRow]; /* [feature][sample] */
+    __shared__ __align__(16) uint16_t F3[64 * kRow]; /* H3, later dZ2 */
+    __shared__ __align__(16) uint16_t F4[64 * kRow]; /* dZ3, later dZ1 */
+    __shared__ __align__(16) uint16_t dz[kChunk];
+    __shared__ float                  yl[kChunk];
+    const int    tid = threadIdx.x, w = tid >> 6, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int    row = 16 * w + 4 * g; /* this lane's four output features */
+    const bf16x4 zero4 = {0, 0, 0, 0}, ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};
+    const f32x4  zacc = {0.f, 0.f, 0.f, 0.f};
+    bf16x4       w1[3], w2[4], w3[4], w4[4], t2[4], t3[4], t4 = zero4;
+    for (int kb = 0; kb < 3; kb++) w1[kb] = *reinterpret_cast<const bf16x4*>(W + kP1 + (16 * w + r) * 48 + 16 * kb + 4 * g);
+    for (int kb = 0; kb < 4; kb++) {
+        const int at = (16 * w + r) * 64 + 16 * kb + 4 * g;
+        w2[kb] = *reinterpret_cast<const bf16x4*>(W + kP2 + at);
+        w3[kb] = *reinterpret_cast<const bf16x4*>(W + kP3 + at);
+        t2[kb] = *reinterpret_cast<const bf16x4*>(W + kPT2 + at);
+        t3[kb] = *reinterpret_cast<const bf16x4*>(W + kPT3 + at);
+        w4[kb] = *reinterpret_cast<const bf16x4*>(W + kP4 + r * 64 + 16 * kb + 4 * g); /* the output row block */
     }
-    TrainFrags F;
-    load_train_frags(W, r, g, F);
-    float* const  row    = gp + (size_t) blockIdx.x * kGradN;
-    const int     chunks = (B + kChunk - 1) / kChunk;
-    double        lsum   = 0.0;
-    const bf16x4  zero4  = {0, 0, 0, 0};
+    t4[0] = g == 0 ? (short) W[kP4 + 16 * w + r] : (short) 0; /* W4^T: one column that is not zero */
+    float b1[4], b2[4], b3[4];
+    for (int e = 0; e < 4; e++) b1[e] = P[kB1 + row + e], b2[e] = P[kB2 + row + e], b3[e] = P[kB3 + row + e];
+    const float b4 = P[kB4];
+    f32x4       g1[3], g2[4], g3[4], g4 = zacc, gb1 = zacc, gb2 = zacc, gb3 = zacc; /* gradients of this wave's rows */
+    for (int t = 0; t < 3; t++) g1[t] = zacc;
+    for (int t = 0; t < 4; t++) g2[t] = g3[t] = zacc;
+    float     gb4    = 0.0f;
+    double    lsum   = 0.0;
+    const int chunks = (T.B + kChunk - 1) / kChunk;
+    /* one layer: rows of the wave, four sample groups: input fragments from
+     * `in` ([sample][feature]), results to `out` and to feat ([feature][sample]) */
+    auto put = [&](uint16_t* out, uint16_t* feat, int j, bf16x4 v) {
+        if (out) lds4(out + (16 * j + r) * kRow + row, v);
+        for (int e = 0; e < 4; e++) feat[(row + e) * kRow + 16 * j + r] = (uint16_t) v[e];
+    };
+    auto dot = [&](const bf16x4* a, int kbs, const uint16_t* in, int j) {
+        f32x4 acc = zacc;
+        for (int kb = 0; kb < kbs; kb++) acc = mfma16(a[kb], lds4(in + (16 * j + r) * kRow + 16 * kb + 4 * g), acc);
+        return acc;
+    };
+    /* rows of a weight gradient: A = the wave's rows of dZ, B = rows of H, K = samples; and the bias's */
+    auto grad = [&](const uint16_t* dZ, const uint16_t* H, int tiles, f32x4* acc, f32x4& gb) {
+        for (int j = 0; j < kChunk / 16; j++) {
+            const bf16x4 a = lds4(dZ + (16 * w + r) * kRow + 16 * j + 4 * g);
+            for (int t = 0; t < tiles; t++) acc[t] = mfma16(a, lds4(H + (16 * t + r) * kRow + 16 * j + 4 * g), acc[t]);
+            gb = mfma16(a, ones, gb);
+        }
+    };
     for (int c = blockIdx.x; c < chunks; c += gridDim.x) {
-        const bool first = c == (int) blockIdx.x;
-        const int  base  = c * kChunk;
-        for (int i = tid; i < kMlpInPad * kChunk; i += blockDim.x) {
-            const int f = i / kChunk, s = base + i % kChunk;
-            L.x[i]      = s < B ? X[(size_t) f * B + s] : (uint16_t) 0;
-        }
-        __syncthreads();
-        const int j = wv; /* this wave's fragment group */
-        if (base + 16 * j >= B) { /* past the batch: zeros, which add nothing below */
-            for (int t = 0; t < 4; t++) {
-                put_frag(L.h1, t, j, zero4, r, g), put_frag(L.h2, t, j, zero4, r, g);
-                put_frag(L.h3, t, j, zero4, r, g), put_frag(L.d1, t, j, zero4, r, g);
-                put_frag(L.d2, t, j, zero4, r, g), put_frag(L.d3, t, j, zero4, r, g);
+        const int base = c * kChunk, s = base + lane;
+        /* features 12 w .. 12 w + 11 of sample `lane` */
+        if (STORE) {
+            float u[3] = {0.f, 0.f, 0.f}, nn[3] = {0.f, 0.f, 0.f}, lu[3] = {0.f, 0.f, 0.f};
+            if (s < T.B) {
+                const RawSample q = T.S[T.perm[T.off + (size_t) s]];
+                mlp_scale(q.isp, T.bx, T.by, T.bz, T.bw, u);
+                mlp_scale(q.light, T.bx, T.by, T.bz, T.bw, lu);
+                nn[0] = q.nrm[0], nn[1] = q.nrm[1], nn[2] = q.nrm[2];
+                if (w == 0) yl[lane] = q.label;
             }
-            put_frag(L.d4, 0, j, zero4, r, g);
+            for (int p = 0; p < 6; p++) {
+                const int f = 12 * w + 2 * p; /* uniform over the wave */
+                float     a, b;
+                if (f < 36) band_sincos(f / 6, pick3(u, (f % 6) >> 1), &a, &b);
+                else a = mlp_feature(f, u, nn, lu), b = mlp_feature(f + 1, u, nn, lu);
+                const uint16_t ab = s < T.B ? f2bf(a) : (uint16_t) 0, bb = s < T.B ? f2bf(b) : (uint16_t) 0;
+                S0[lane * kRow + f]       = ab;
+                S0[lane * kRow + f + 1]   = bb;
+                Xf[f * kRow + lane]       = ab;
+                Xf[(f + 1) * kRow + lane] = bb;
+            }
         } else {
-            /* forward */
-            bf16x4 xin[3], h1[4], h2[4], h3[4];
-            for (int kb = 0; kb < 3; kb++)
-                for (int e = 0; e < 4; e++) xin[kb][e] = (short) L.x[(16 * kb + 4 * g + e) * kChunk + 16 * j + r];
-            for (int mt = 0; mt < 4; mt++) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                for (int kb = 0; kb < 3; kb++) acc = mfma16(F.w1[mt][kb], xin[kb], acc);
-                h1[mt] = relu_pack(acc, L.bias + kLB1 + 16 * mt + 4 * g);
-                put_frag(L.h1, mt, j, h1[mt], r, g);
+            for (int f = 12 * w; f < 12 * w + 12; f++) {
+                const uint16_t v     = s < T.B ? T.X[(size_t) f * T.B + s] : (uint16_t) 0;
+                S0[lane * kRow + f]  = v;
+                Xf[f * kRow + lane]  = v;
             }
-            for (int mt = 0; mt < 4; mt++) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                for (int kb = 0; kb < 4; kb++) acc = mfma16(F.w2[mt][kb], h1[kb], acc);
-                h2[mt] = relu_pack(acc, L.bias + kLB2 + 16 * mt + 4 * g);
-                put_frag(L.h2, mt, j, h2[mt], r, g);
-            }
-            for (int mt = 0; mt < 4; mt++) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                for (int kb = 0; kb < 4; kb++) acc = mfma16(F.w3[mt][kb], h2[kb], acc);
-                h3[mt] = relu_pack(acc, L.bias + kLB3 + 16 * mt + 4 * g);
-                put_frag(L.h3, mt, j, h3[mt], r, g);
-            }
-            f32x4 lg = {0.f, 0.f, 0.f, 0.f};
-            for (int kb = 0; kb < 4; kb++) lg = mfma16(F.w4[kb], h3[kb], lg);
-            /* loss and output gradient: row 0 of the output tile, lanes 0..15 */
-            const int s  = base + 16 * j + r;
-            float     dz = 0.0f;
-            if (g == 0 && s < n) {
-                const float p  = 1.0f / (1.0f + expf(-(lg[0] + L.bias[kLB4])));
-                const float y  = Y[s];
-                const float pc = fminf(fmaxf(p, 1e-7f), 1.0f - 1e-7f);
-                lsum += y > 0.5f ? -log((double) pc) : -log(1.0 - (double) pc);
-                dz = (p - y) / (float) n;
-            }
-            bf16x4 d4 = zero4;
-            d4[0]     = g == 0 ? (short) f2bf(dz) : (short) 0; /* row 0 of dZ4; rows 1..15 zero */
-            put_frag(L.d4, 0, j, d4, r, g);
-            /* backward */
-            bf16x4 d3[4], d2[4];
-            for (int mt = 0; mt < 4; mt++) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                acc       = mfma16(F.t4[mt], d4, acc);
-                d3[mt]    = mask_pack(acc, h3[mt]);
-                put_frag(L.d3, mt, j, d3[mt], r, g);
-            }
-            for (int mt = 0; mt < 4; mt++) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                for (int kb = 0; kb < 4; kb++) acc = mfma16(F.t3[mt][kb], d3[kb], acc);
-                d2[mt] = mask_pack(acc, h2[mt]);
-                put_frag(L.d2, mt, j, d2[mt], r, g);
-            }
-            for (int mt = 0; mt < 4; mt++) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                for (int kb = 0; kb < 4; kb++) acc = mfma16(F.t2[mt][kb], d2[kb], acc);
-                put_frag(L.d1, mt, j, mask_pack(acc, h1[mt]), r, g);
-            }
+            if (w == 0) yl[lane] = s < T.B ? T.Y[s] : 0.0f;
         }
         __syncthreads();
-        /* weight gradients of the chunk, dW_l = dZ_l H_{l-1}^T: 48 tiles, wave w takes w, w + 4, ... */
-        for (int t = wv; t < 48; t += 4) {
-            if (t < 12) {
-                const int mt = t / 3, nt = t % 3;
-                add_tile(row, first, kP1, 48, mt, nt, chunk_tile(L.d1, L.x, mt, nt, r, g), r, g);
-            } else if (t < 28) {
-                const int mt = (t - 12) / 4, nt = (t - 12) % 4;
-                add_tile(row, first, kP2, 64, mt, nt, chunk_tile(L.d2, L.h1, mt, nt, r, g), r, g);
-            } else if (t < 44) {
-                const int mt = (t - 28) / 4, nt = (t - 28) % 4;
-                add_tile(row, first, kP3, 64, mt, nt, chunk_tile(L.d3, L.h2, mt, nt, r, g), r, g);
-            } else {
-                const int nt = t - 44;
-                add_tile(row, first, kP4, 64, 0, nt, chunk_tile(L.d4, L.h3, 0, nt, r, g), r, g);
+        bf16x4 h1[4], h2[4], h3[4];
+        for (int j = 0; j < 4; j++) put(S1, H1, j, h1[j] = relu_pack(dot(w1, 3, S0, j), b1));
+        __syncthreads();
+        for (int j = 0; j < 4; j++) put(S0, H2, j, h2[j] = relu_pack(dot(w2, 4, S1, j), b2));
+        __syncthreads();
+        for (int j = 0; j < 4; j++) put(S1, F3, j, h3[j] = relu_pack(dot(w3, 4, S0, j), b3));
+        __syncthreads();
+        { /* loss and output gradient of sample group w: row 0 of the output tile, lanes 0..15 */
+            const f32x4 lg = dot(w4, 4, S1, w);
+            const int   q  = base + 16 * w + r;
+            float       d  = 0.0f;
+            if (g == 0 && q < T.n) {
+                const float p = 1.0f / (1.0f + expf(-(lg[0] + b4)));
+                const float y = yl[16 * w + r];
+                if (loss) {
+                    const float pc = fminf(fmaxf(p, 1e-7f), 1.0f - 1e-7f);
+                    lsum += y > 0.5f ? -log((double) pc) : -log(1.0 - (double) pc);
+                }
+                d = (p - y) / (float) T.n;
             }
+            if (g == 0) dz[16 * w + r] = f2bf(d);
         }
-        /* bias gradients: row sums, wave w takes layer w + 1 (lane = feature) */
-        if (wv < 3 || lane == 0) {
-            const uint16_t* d   = wv == 0 ? L.d1 : wv == 1 ? L.d2 : wv == 2 ? L.d3 : L.d4;
-            const int       off = wv == 0 ? kGB1 : wv == 1 ? kGB2 : wv == 2 ? kGB3 : kGB4;
-            float           acc = 0.0f;
-            for (int k = 0; k < kChunk; k++) acc += bf2f(d[lane * kChunk + k]);
-            row[off + lane] = first ? acc : row[off + lane] + acc;
+        __syncthreads();
+        for (int j = 0; j < 4; j++) {
+            bf16x4 d4 = zero4; /* row 0 of dZ4; rows 1..15 zero */
+            d4[0]     = g == 0 ? (short) dz[16 * j + r] : (short) 0;
+            put(S0, F4, j, mask_pack(mfma16(t4, d4, zacc), h3[j]));
+            const bf16x4 a4 = r == 0 ? lds4(dz + 16 * j + 4 * g) : zero4; /* dW4: columns 16 w .. of its row 0 */
+            g4 = mfma16(a4, lds4(F3 + (16 * w + r) * kRow + 16 * j + 4 * g), g4);
         }
+        if (w == 0) gb4 += bf2f(dz[lane]);
+        __syncthreads();
+        for (int j = 0; j < 4; j++) put(S1, F3, j, mask_pack(dot(t3, 4, S0, j), h2[j]));
+        grad(F4, H2, 4, g3, gb3);
+        __syncthreads();
+        for (int j = 0; j < 4; j++) put(nullptr, F4, j, mask_pack(dot(t2, 4, S1, j), h1[j]));
+        grad(F3, H1, 4, g2, gb2);
+        __syncthreads();
+        grad(F4, Xf, 3, g1, gb1);
         __syncthreads(); /* the next chunk overwrites the LDS arrays */
     }
-    for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
-    if (lane == 0 && lsum != 0.0) atomicAdd(loss, lsum);
+    float* const out = gp + (size_t) blockIdx.x * kGradN;
+    for (int t = 0; t < 3; t++) *reinterpret_cast<f32x4*>(out + 256 * (3 * w + t) + 4 * lane) = g1[t];
+    for (int t = 0; t < 4; t++) *reinterpret_cast<f32x4*>(out + kG2 + 256 * (4 * w + t) + 4 * lane) = g2[t];
+    for (int t = 0; t < 4; t++) *reinterpret_cast<f32x4*>(out + kG3 + 256 * (4 * w + t) + 4 * lane) = g3[t];
+    if (g == 0) out[kG4 + 16 * w + r] = g4[0];
+    if (r == 0) { /* every column of these is the same sum */
+        *reinterpret_cast<f32x4*>(out + kGB1 + row) = gb1;
+        *reinterpret_cast<f32x4*>(out + kGB2 + row) = gb2;
+        *reinterpret_cast<f32x4*>(out + kGB3 + row) = gb3;
+    }
+    if (w == 0) {
+        for (int o = 32; o > 0; o >>= 1) gb4 += __shfl_xor(gb4, o, 64);
+        if (lane == 0) out[kGB4] = gb4;
+    }
+    if (loss) {
+        for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
+        if (lane == 0 && lsum != 0.0) atomicAdd(loss, lsum);
+    }
 }
 
-/* G[i] = sum over the rows of the partial gradients */
-__global__ void k_grad_rows(const float* __restrict__ gp, int rows, float* __restrict__ G)
+/* partial-gradient element -> flat parameter index (-1: padding), and where
+ * the weight's bf16 copies sit (pk; pt, W2 and W3 only) */
+__device__ __forceinline__ int grad_param(int i, int& pk, int& pt)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= kGradN) return;
-    float acc = 0.0f;
-    for (int b = 0; b < rows; b++) acc += gp[(size_t) b * kGradN + i];
-    G[i] = acc;
+    pk = pt = -1;
+    if (i < kG4) {
+        const int t = i < kG2 ? i / 256 : (i < kG3 ? i - kG2 : i - kG3) / 256, nts = i < kG2 ? 3 : 4;
+        const int lane = (i & 255) >> 2, o = 16 * (t / nts) + 4 * (lane >> 4) + (i & 3), c = 16 * (t % nts) + (lane & 15);
+        if (i < kG2) {
+            if (c >= kMlpIn) return -1;
+            pk = kP1 + o * 48 + c;
+            return kW1 + o * kMlpIn + c;
+        }
+        pk = (i < kG3 ? kP2 : kP3) + o * 64 + c;
+        pt = (i < kG3 ? kPT2 : kPT3) + c * 64 + o;
+        return (i < kG3 ? kW2 : kW3) + o * 64 + c;
+    }
+    if (i < kGB1) {
+        pk = kP4 + (i - kG4);
+        return kW4 + (i - kG4);
+    }
+    if (i < kGB2) return kB1 + (i - kGB1);
+    if (i < kGB3) return kB2 + (i - kGB2);
+    if (i < kGB4) return kB3 + (i - kGB3);
+    return i == kGB4 ? kB4 : -1;
 }
 
-/* the 48 (padded) features of a query, bf16, feature-major X[48][B] */
-__device__ __forceinline__ void store_features(uint16_t* __restrict__ X, int B, int s, const float u[3],
-                                               const float nrm[3], const float lu[3])
-{
-    for (int f = 0; f < kMlpInPad; f++) X[(size_t) f * B + s] = f2bf(mlp_feature(f, u, nrm, lu));
-}
+struct AdamArgs {
+    float lr, b1, b2, eps, c1, c2;
+};
 
-/* minibatch from the sample store: X, labels Y */
-__global__ void k_batch_features(const RawSample* __restrict__ S, const uint32_t* __restrict__ perm, size_t off,
-                                 int B, float bx, float by, float bz, float bw, uint16_t* __restrict__ X,
-                                 float* __restrict__ Y)
+/* The sum of the blocks' partial gradients (64 elements per block, four row
+ * groups), then either the gradient in flat order (grads not null), or one
+ * Adam step (Kingma & Ba 2015, bias-corrected moments, fp32 master weights)
+ * and the weights' new bf16 copies. 3.9 us for 64 rows, against 16 + 4.6 +
+ * 4.5 for a sum by one thread per element, Adam and repack as launches. */
+__global__ void __launch_bounds__(256) k_mlp_step(const float* __restrict__ gp, int rows, float* __restrict__ grads,
+                                                  float* __restrict__ P, float* __restrict__ m, float* __restrict__ v,
+                                                  uint16_t* __restrict__ W, AdamArgs A)
 {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= B) return;
-    const RawSample q = S[perm[off + (size_t) s]];
-    float           u[3], lu[3];
-    mlp_scale(q.isp, bx, by, bz, bw, u);
-    mlp_scale(q.light, bx, by, bz, bw, lu);
-    store_features(X, B, s, u, q.nrm, lu);
-    Y[s] = q.label;
+    __shared__ float part[4][64];
+    const int        lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+    const int        per = (rows + 3) / 4, lo = w * per, hi = min(rows, lo + per);
+    float            acc = 0.0f;
+#pragma unroll 8
+    for (int b = lo; b < hi; b++) acc += gp[(size_t) b * kGradN + i];
+    part[w][lane] = acc;
+    __syncthreads();
+    if (w != 0) return;
+    int         pk, pt;
+    const int   p = grad_param(i, pk, pt);
+    const float g = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    if (p < 0) return;
+    if (grads) {
+        grads[p] = g;
+        return;
+    }
+    const float mn = A.b1 * m[p] + (1.0f - A.b1) * g, vn = A.b2 * v[p] + (1.0f - A.b2) * g * g;
+    m[p]           = mn;
+    v[p]           = vn;
+    const float pn = P[p] - A.lr * (mn / A.c1) / (sqrtf(vn / A.c2) + A.eps);
+    P[p]           = pn;
+    if (pk >= 0) W[pk] = f2bf(pn);
+    if (pt >= 0) W[pt] = f2bf(pn);
 }
 
 /* supplied feature rows (n x 42 fp32) -> X; columns n..B-1 zero */
@@ -393,39 +406,6 @@ __global__ void k_copy_features(const float* __restrict__ x, int B, int n, uint1
     for (int f = 0; f < kMlpInPad; f++)
         X[(size_t) f * B + s] = f2bf((s < n && f < kMlpIn) ? x[(size_t) s * kMlpIn + f] : 0.0f);
     if (Y) Y[s] = (s < n && yin) ? yin[s] : 0.0f;
-}
-
-/* flat parameter index -> gradient-layout index */
-__device__ __forceinline__ int grad_index(int i)
-{
-    if (i < kB1) return kP1 + (i / kMlpIn) * 48 + (i % kMlpIn);
-    if (i < kW2) return kGB1 + (i - kB1);
-    if (i < kB2) return kP2 + (i - kW2);
-    if (i < kW3) return kGB2 + (i - kB2);
-    if (i < kB3) return kP3 + (i - kW3);
-    if (i < kW4) return kGB3 + (i - kB3);
-    if (i < kB4) return kP4 + (i - kW4);
-    return kGB4;
-}
-
-/* Adam (Kingma & Ba 2015), bias-corrected moments, fp32 master weights */
-__global__ void k_mlp_adam(float* __restrict__ P, const float* __restrict__ G, float* __restrict__ m,
-                           float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= kMlpParams) return;
-    float g  = G[grad_index(i)];
-    m[i]     = b1 * m[i] + (1.0f - b1) * g;
-    v[i]     = b2 * v[i] + (1.0f - b2) * g * g;
-    float mh = m[i] / c1;
-    float vh = v[i] / c2;
-    P[i]     = P[i] - lr * mh / (sqrtf(vh) + eps);
-}
-
-__global__ void k_grads_to_flat(const float* __restrict__ G, float* __restrict__ out)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < kMlpParams) out[i] = G[grad_index(i)];
 }
 
 /* random sort keys for the sample shuffle */
@@ -779,7 +759,7 @@ void qbt_ctx::mlp_free()
 {
     if (!mlp) return;
     MlpState* m = mlp;
-    for (DevBuf* b : {&m->params, &m->m, &m->v, &m->grads, &m->packed, &m->ctr, &m->samples, &m->perm, &m->keys,
+    for (DevBuf* b : {&m->params, &m->m, &m->v, &m->packed, &m->ctr, &m->samples, &m->perm, &m->keys,
                       &m->vals, &m->sort_tmp, &m->X, &m->gpart, &m->lossbuf, &m->io_x, &m->io_p, &m->io_y,
                       &m->io_a, &m->io_c, &m->flat})
         dev_free(*b);
@@ -797,8 +777,7 @@ static int mlp_state(qbt_ctx* c, MlpState** out)
         MlpState* m = c->mlp;
         int       rc;
         if ((rc = c->dev_alloc(m->params, kMlpParams * 4)) || (rc = c->dev_alloc(m->m, kMlpParams * 4)) ||
-            (rc = c->dev_alloc(m->v, kMlpParams * 4)) || (rc = c->dev_alloc(m->grads, kGradN * 4)) ||
-            (rc = c->dev_alloc(m->packed, kPackN * 2)) || (rc = c->dev_alloc(m->lossbuf, 64)) ||
+            (rc = c->dev_alloc(m->v, kMlpParams * 4)) || (rc = c->dev_alloc(m->packed, kPackAll * 2)) || (rc = c->dev_alloc(m->lossbuf, 64)) ||
             (rc = c->dev_alloc(m->ctr, 16)) || (rc = c->dev_alloc(m->flat, kMlpParams * 4))) {
             c->mlp_free();
             return rc;
@@ -812,7 +791,7 @@ static int mlp_state(qbt_ctx* c, MlpState** out)
 
 static int mlp_repack(qbt_ctx* c)
 {
-    k_mlp_pack<<<nblk(kPackN), 256, 0, c->stream>>>((const float*) c->mlp->params.p, (uint16_t*) c->mlp->packed.p);
+    k_mlp_pack<<<nblk(kPackAll), 256, 0, c->stream>>>((const float*) c->mlp->params.p, (uint16_t*) c->mlp->packed.p);
     HIPCHK(hipGetLastError());
     return QBT_OK;
 }
@@ -934,64 +913,59 @@ extern "C" int qbt_surrogate_read_samples(qbt_ctx* c, size_t start, size_t n, fl
 
 constexpr int kTrainBlocks = 256; /* blocks of k_mlp_train, rows of partial gradients, at most */
 
-/* batch buffers for batch width B (multiple of 16) */
-static int mlp_batch_bufs(qbt_ctx* c, int B)
-{
-    MlpState*    m      = c->mlp;
-    const size_t b      = (size_t) B;
-    const size_t chunks = (b + kChunk - 1) / kChunk;
-    const size_t rows   = chunks < (size_t) kTrainBlocks ? chunks : (size_t) kTrainBlocks;
-    int          rc;
-    if ((rc = c->dev_alloc(m->X, kMlpInPad * b * 2)) || (rc = c->dev_alloc(m->gpart, rows * kGradN * 4)) ||
-        (rc = c->dev_alloc(m->io_y, b * 4)) || (rc = c->dev_alloc(m->io_p, b * 4)))
-        return rc;
-    return QBT_OK;
-}
+static int train_rows(int B) { return std::min((B + kChunk - 1) / kChunk, kTrainBlocks); }
 
-/* Forward and backward of the B-column batch in X (n valid columns, labels
- * in io_y): the summed loss into lossbuf, the gradient (layout kGradN) into
- * grads. Three launches: loss reset, k_mlp_train, k_grad_rows. */
-static int mlp_fwd_bwd(qbt_ctx* c, int B, int n, double* loss_out)
+/* the partial gradients of a batch of width B */
+static int mlp_grad_buf(qbt_ctx* c, int B) { return c->dev_alloc(c->mlp->gpart, (size_t) train_rows(B) * kGradN * 4); }
+
+/* Forward and backward of a minibatch: the partial gradients into gpart and,
+ * if asked for, the summed loss into lossbuf. */
+static int mlp_fwd_bwd(qbt_ctx* c, const TrainBatch& T, bool want_loss)
 {
-    MlpState*   m      = c->mlp;
-    hipStream_t st     = c->stream;
-    const int   chunks = (B + kChunk - 1) / kChunk;
-    const int   rows   = chunks < kTrainBlocks ? chunks : kTrainBlocks;
-    double*     lossd  = (double*) m->lossbuf.p;
-    k_fill_f32<<<1, 64, 0, st>>>((float*) m->lossbuf.p, 2, 0.0f);
-    k_mlp_train<<<rows, 256, 0, st>>>((const uint16_t*) m->packed.p, (const float*) m->params.p,
-                                      (const uint16_t*) m->X.p, (const float*) m->io_y.p, B, n, (float*) m->gpart.p,
-                                      lossd);
-    k_grad_rows<<<nblk(kGradN), 256, 0, st>>>((const float*) m->gpart.p, rows, (float*) m->grads.p);
+    MlpState*       m    = c->mlp;
+    const int       rows = train_rows(T.B);
+    double*         loss = want_loss ? (double*) m->lossbuf.p : nullptr;
+    const uint16_t* W    = (const uint16_t*) m->packed.p;
+    if (loss) k_fill_f32<<<1, 64, 0, c->stream>>>((float*) m->lossbuf.p, 2, 0.0f);
+    if (T.S) k_mlp_train<true><<<rows, 256, 0, c->stream>>>(W, (const float*) m->params.p, T, (float*) m->gpart.p, loss);
+    else k_mlp_train<false><<<rows, 256, 0, c->stream>>>(W, (const float*) m->params.p, T, (float*) m->gpart.p, loss);
     HIPCHK(hipGetLastError());
-    if (loss_out) {
-        double l = 0.0;
-        HIPCHK(hipMemcpyAsync(&l, lossd, 8, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        *loss_out = l / (n > 0 ? n : 1);
-    }
     return QBT_OK;
 }
 
-static int mlp_adam_step(qbt_ctx* c, float lr)
+/* mean loss of the last mlp_fwd_bwd that was asked for it (synchronises) */
+static int mlp_read_loss(qbt_ctx* c, int n, double* out)
+{
+    double l = 0.0;
+    HIPCHK(hipMemcpyAsync(&l, c->mlp->lossbuf.p, 8, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    *out = l / (n > 0 ? n : 1);
+    return QBT_OK;
+}
+
+/* an Adam step with the gradient of the last mlp_fwd_bwd (batch width B) */
+static int mlp_adam_step(qbt_ctx* c, int B, float lr)
 {
     MlpState* m = c->mlp;
     m->t++;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const float c1 = 1.0f - powf(b1, (float) m->t), c2 = 1.0f - powf(b2, (float) m->t);
-    k_mlp_adam<<<nblk(kMlpParams), 256, 0, c->stream>>>((float*) m->params.p, (const float*) m->grads.p,
-                                                         (float*) m->m.p, (float*) m->v.p, lr, b1, b2, eps, c1, c2);
+    k_mlp_step<<<kGradN / 64, 256, 0, c->stream>>>((const float*) m->gpart.p, train_rows(B), nullptr, (float*) m->params.p,
+                                                   (float*) m->m.p, (float*) m->v.p, (uint16_t*) m->packed.p,
+                                                   AdamArgs{lr, b1, b2, eps, c1, c2});
     HIPCHK(hipGetLastError());
-    return mlp_repack(c);
+    return QBT_OK;
 }
 
 /* host feature rows (n x 42) -> X, labels -> io_y; B = n rounded up to 16 */
 static int mlp_load_host(qbt_ctx* c, const float* x, const float* y, size_t n, int* Bout)
 {
     MlpState* m = c->mlp;
-    const int B = (int) ((n + 15) / 16) * 16;
-    int       rc;
-    if ((rc = mlp_batch_bufs(c, B)) || (rc = c->dev_alloc(m->io_x, n * kMlpIn * 4)) ||
+    const int    B = (int) ((n + 15) / 16) * 16;
+    const size_t b = (size_t) B;
+    int          rc;
+    if ((rc = c->dev_alloc(m->X, kMlpInPad * b * 2)) || (rc = c->dev_alloc(m->io_y, b * 4)) ||
+        (rc = c->dev_alloc(m->io_p, b * 4)) || (rc = c->dev_alloc(m->io_x, n * kMlpIn * 4)) ||
         (rc = c->dev_alloc(m->io_a, n * 4)))
         return rc;
     HIPCHK(hipMemcpyAsync(m->io_x.p, x, n * kMlpIn * 4, hipMemcpyHostToDevice, c->stream));
@@ -1053,31 +1027,41 @@ extern "C" int qbt_surrogate_predict(qbt_ctx* c, const float* isp, const float* 
     return QBT_OK;
 }
 
-extern "C" int qbt_surrogate_grad(qbt_ctx* c, const float* x, const float* y, size_t n, float* grads, float* loss)
+/* forward and backward of n labelled host rows; *B the padded batch width */
+static int mlp_host_batch(qbt_ctx* c, const float* x, const float* y, size_t n, float* loss, int* B)
 {
     if (!c || !x || !y || n == 0 || n > ((size_t) 1 << 22) || !qbt_surrogate_ready(c)) return QBT_EINVAL;
     HIPCHK(hipSetDevice(c->device));
-    int B, rc;
-    if ((rc = mlp_load_host(c, x, y, n, &B))) return rc;
+    int rc;
+    if ((rc = mlp_load_host(c, x, y, n, B)) || (rc = mlp_grad_buf(c, *B))) return rc;
+    TrainBatch T{};
+    T.X = (const uint16_t*) c->mlp->X.p, T.Y = (const float*) c->mlp->io_y.p, T.B = *B, T.n = (int) n;
+    if ((rc = mlp_fwd_bwd(c, T, true))) return rc;
     double l = 0.0;
-    if ((rc = mlp_fwd_bwd(c, B, (int) n, &l))) return rc;
-    if (grads) {
-        k_grads_to_flat<<<nblk(kMlpParams), 256, 0, c->stream>>>((const float*) c->mlp->grads.p,
-                                                                  (float*) c->mlp->flat.p);
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(grads, c->mlp->flat.p, kMlpParams * 4, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-    }
+    if ((rc = mlp_read_loss(c, (int) n, &l))) return rc;
     if (loss) *loss = (float) l;
+    return QBT_OK;
+}
+
+extern "C" int qbt_surrogate_grad(qbt_ctx* c, const float* x, const float* y, size_t n, float* grads, float* loss)
+{
+    int B, rc;
+    if ((rc = mlp_host_batch(c, x, y, n, loss, &B))) return rc;
+    if (!grads) return QBT_OK;
+    MlpState* m = c->mlp;
+    k_mlp_step<<<kGradN / 64, 256, 0, c->stream>>>((const float*) m->gpart.p, train_rows(B), (float*) m->flat.p, nullptr,
+                                                   nullptr, nullptr, nullptr, AdamArgs{});
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(grads, m->flat.p, kMlpParams * 4, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
     return QBT_OK;
 }
 
 extern "C" int qbt_surrogate_step(qbt_ctx* c, const float* x, const float* y, size_t n, float lr, float* loss)
 {
     if (!(lr >= 0.0f)) return QBT_EINVAL;
-    int rc = qbt_surrogate_grad(c, x, y, n, nullptr, loss);
-    if (rc) return rc;
-    if ((rc = mlp_adam_step(c, lr))) return rc;
+    int B, rc;
+    if ((rc = mlp_host_batch(c, x, y, n, loss, &B)) || (rc = mlp_adam_step(c, B, lr))) return rc;
     HIPCHK(hipStreamSynchronize(c->stream));
     return QBT_OK;
 }
@@ -1114,7 +1098,7 @@ extern "C" int qbt_surrogate_train(qbt_ctx* c, const float basecube[4], int step
     int       rc;
     if ((rc = mlp_counts(c, &n, nullptr))) return rc;
     if (n < (size_t) batch) return QBT_EINVAL;
-    if ((rc = mlp_batch_bufs(c, batch)) || (rc = c->dev_alloc(m->perm, n * 4)) || (rc = c->dev_alloc(m->keys, n * 8)) ||
+    if ((rc = mlp_grad_buf(c, batch)) || (rc = c->dev_alloc(m->perm, n * 4)) || (rc = c->dev_alloc(m->keys, n * 8)) ||
         (rc = c->dev_alloc(m->vals, n * 4)))
         return rc;
     size_t tb = 0;
@@ -1133,19 +1117,17 @@ extern "C" int qbt_surrogate_train(qbt_ctx* c, const float basecube[4], int step
     };
     /* a new shuffle when the store changed size or the permutation is used up */
     if (m->perm_n != n && (rc = shuffle())) return rc;
-    double last = 0.0;
     for (int it = 0; it < steps; it++) {
         if (m->pos + (size_t) batch > n && (rc = shuffle())) return rc;
-        k_batch_features<<<nblk(batch), 256, 0, c->stream>>>((const RawSample*) m->samples.p,
-                                                             (const uint32_t*) m->perm.p, m->pos, batch, basecube[0],
-                                                             basecube[1], basecube[2], basecube[3],
-                                                             (uint16_t*) m->X.p, (float*) m->io_y.p);
-        HIPCHK(hipGetLastError());
+        TrainBatch T{};
+        T.S = (const RawSample*) m->samples.p, T.perm = (const uint32_t*) m->perm.p, T.off = m->pos;
+        T.bx = basecube[0], T.by = basecube[1], T.bz = basecube[2], T.bw = basecube[3];
+        T.B = T.n = batch;
         m->pos += (size_t) batch;
-        if ((rc = mlp_fwd_bwd(c, batch, batch, it == steps - 1 ? &last : nullptr))) return rc;
-        if ((rc = mlp_adam_step(c, lr))) return rc;
+        if ((rc = mlp_fwd_bwd(c, T, it == steps - 1)) || (rc = mlp_adam_step(c, batch, lr))) return rc;
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
+    double last = 0.0;
+    if ((rc = mlp_read_loss(c, batch, &last))) return rc;
     if (loss_out) *loss_out = (float) last;
     return QBT_OK;
 }

@@ -113,7 +113,12 @@ __device__ __forceinline__ uint32_t* wave_mail(uint32_t* lds, int L)
 /* Camera rays of the batch. Work items 0 .. nspr-1 are the sprite traces
  * (view i / nl, light i % nl: the ray from the camera to the light,
  * octree_fsh.c:452-459, one per view and light; result flags to
- * b.sprite), then nitems pixel items. */
+ * b.sprite), then nitems pixel items.
+ *
+ * Bound by the issue of the traversal step's vector instructions and, towards
+ * the end, by the latency of a lone wave's step. Five waves per SIMD (91
+ * VGPRs): at six the slow paths spill, and 2.07M short rays take 352 us
+ * against 328 (long ones, 8.3M of a 2160p frame, 6.32 against 6.49 ms). */
 template <bool CMP, bool DUAL, bool GRID, bool COUNT, bool GSTK>
 __global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, PrimOut o, uint32_t nitems, uint32_t nspr,
                                                  int nl, int strip, int* __restrict__ sprite, unsigned* __restrict__ q,
@@ -126,22 +131,33 @@ __global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, Prim
     const Stack st   = lane_stack<DUAL, GSTK>(lds, gstack, s.maxlevel);
     const int   lane = threadIdx.x & 63;
     bool        active = false;
-    uint32_t    item = 0, gp = 0;
-    int         spr  = -1; /* sprite slot of a sprite lane */
+    uint32_t    k      = 0; /* the lane's work item: a sprite trace below nspr, else camera item k - nspr */
     Ray         r = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     TraceState  t;
     unsigned    n_exp = 0, n_abort = 0, n_hit = 0;
 
+    /* the item's view and pixel; false for the padding of an edge tile. Done
+     * again at the end of the ray: kept in registers they spilled (12 bytes
+     * at 5 waves) */
+    auto pixel = [&](uint32_t it, int& v, int& px, int& py) {
+        v               = batch_view(b.item_off, b.n, it);
+        const ViewDev& V = b.views[v];
+        return item_pixel(it - b.item_off[v], V.w, V.h, strip, px, py);
+    };
+
     auto finish = [&](int stt) {
-        if (spr >= 0) { /* white if the light is in front of the first surface (resv / lghtv.x > 1) */
+        if (k < nspr) { /* white if the light is in front of the first surface (resv / lghtv.x > 1) */
             const float ix = stt == ST_HIT ? t.entry.x : 0.0f;
             int         f  = 0;
             if (stt == ST_DISCARD) f |= 1;
             if ((ix - r.px) / r.dx > 1.0f) f |= 2;
             if (stt == ST_ABORT) f |= 4;
-            sprite[spr] = f;
+            sprite[(k / (uint32_t) nl) * kNL + k % (uint32_t) nl] = f;
             return;
         }
+        int v, px, py;
+        (void) pixel(k - nspr, v, px, py);
+        const uint32_t gp = b.pix_off[v] + (uint32_t) py * (uint32_t) b.views[v].w + (uint32_t) px;
         float4   isp = make_float4(0.f, 0.f, 0.f, 0.f);
         int      ms = -1, md = -1, leaf = -1;
         uint8_t  f    = 0;
@@ -164,12 +180,12 @@ __global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, Prim
                 cand = gp;
             }
         }
-        o.isp[gp]    = isp;
-        o.ms[gp]     = ms;
-        o.md[gp]     = md;
-        o.leaf[gp]   = leaf;
-        o.flags[gp]  = f;
-        o.cand[item] = cand;
+        o.isp[gp]        = isp;
+        o.ms[gp]         = ms;
+        o.md[gp]         = md;
+        o.leaf[gp]       = leaf;
+        o.flags[gp]      = f;
+        o.cand[k - nspr] = cand;
         if (COUNT) {
             o.exp[gp] = (int) t.exps;
             n_exp += t.exps;
@@ -188,41 +204,39 @@ __global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, Prim
         if (given || (rf.left > 0 && (__popcll(idle) >= (int) refill || idle == ~0ull))) {
             const uint32_t fetched = given ? first : rf.fetch(&q[Q_PRIM], idle, lane);
             given                  = false;
-            if (fetched != UINT32_MAX && fetched < nspr) {
-                const int      v = (int) (fetched / (uint32_t) nl), l = (int) (fetched % (uint32_t) nl);
-                const ViewDev& V = b.views[v];
-                spr              = v * kNL + l;
-                r.px             = V.cam[0];
-                r.py             = V.cam[1];
-                r.pz             = V.cam[2];
-                r.dx             = V.light[l][0] - V.cam[0];
-                r.dy             = V.light[l][1] - V.cam[1];
-                r.dz             = V.light[l][2] - V.cam[2];
-                int stt          = trace_begin<false>(s, r, t);
-                if (stt == ST_CONT) active = true;
-                else finish(stt);
-            } else if (fetched != UINT32_MAX) {
-                const uint32_t it = fetched - nspr;
-                const int      v  = batch_view(b.item_off, b.n, it);
-                const ViewDev& V  = b.views[v];
-                int            px, py;
-                item = it;
-                spr  = -1;
-                if (item_pixel(it - b.item_off[v], V.w, V.h, strip, px, py)) {
-                    gp = b.pix_off[v] + (uint32_t) py * (uint32_t) V.w + (uint32_t) px;
-                    float csv[3];
-                    pixel_dir(V, px, py, csv);
-                    r.px    = V.cam[0];
-                    r.py    = V.cam[1];
-                    r.pz    = V.cam[2];
-                    r.dx    = csv[0];
-                    r.dy    = csv[1];
-                    r.dz    = csv[2];
-                    int stt = trace_begin<false>(s, r, t);
+            if (fetched != UINT32_MAX) {
+                bool ray = true;
+                k        = fetched;
+                if (k < nspr) {
+                    const int      v = (int) (k / (uint32_t) nl), l = (int) (k % (uint32_t) nl);
+                    const ViewDev& V = b.views[v];
+                    r.px             = V.cam[0];
+                    r.py             = V.cam[1];
+                    r.pz             = V.cam[2];
+                    r.dx             = V.light[l][0] - V.cam[0];
+                    r.dy             = V.light[l][1] - V.cam[1];
+                    r.dz             = V.light[l][2] - V.cam[2];
+                } else {
+                    int v, px, py;
+                    ray = pixel(k - nspr, v, px, py);
+                    if (ray) {
+                        const ViewDev& V = b.views[v];
+                        float          csv[3];
+                        pixel_dir(V, px, py, csv);
+                        r.px = V.cam[0];
+                        r.py = V.cam[1];
+                        r.pz = V.cam[2];
+                        r.dx = csv[0];
+                        r.dy = csv[1];
+                        r.dz = csv[2];
+                    } else {
+                        o.cand[k - nspr] = UINT32_MAX; /* padding item of an edge tile */
+                    }
+                }
+                if (ray) {
+                    const int stt = trace_begin<false>(s, r, t);
                     if (stt == ST_CONT) active = true;
                     else finish(stt);
-                } else {
-                    o.cand[it] = UINT32_MAX; /* padding item of an edge tile */
                 }
             }
         }
@@ -467,9 +481,14 @@ __global__ void k_oct_scan(const unsigned* __restrict__ cnt, unsigned* __restric
  * has already discarded; otherwise it is traced as well: k_shade stops at the
  * first discarding light, for the colour, the bits and the expansion count
  * (lexp: per light, counting renders), so the frame does not depend on the
- * order in which rays end (the sample collector applies the same rule). */
+ * order in which rays end (the sample collector applies the same rule).
+ *
+ * Five waves per SIMD (95 VGPRs) against six, which spill: 536 against 560
+ * us on the shadow rays of a 1080p frame of 10M points, 1.82 against 1.87 ms
+ * on a batch of 12 views; 8.58 against 8.49 ms on a 2160p frame of 30M. */
 template <bool CMP, bool DUAL, bool GRID, bool COUNT, bool GSTK>
-__global__ void __launch_bounds__(256, DUAL ? 5 : 6) k_shadow(SceneDev s, LightsDev L, const uint32_t* __restrict__ lists,
+__global__ void __launch_bounds__(256, 5)
+    k_shadow(SceneDev s, LightsDev L, const uint32_t* __restrict__ lists,
                                                 size_t lstride, const unsigned* __restrict__ counts, int cstride,
                                                 const float4* __restrict__ isp, uint8_t* __restrict__ lstat,
                                                 size_t npix, unsigned* __restrict__ disc, unsigned* __restrict__ q,
@@ -617,8 +636,9 @@ __device__ __forceinline__ uint32_t slot_xchg(uint32_t* p, uint32_t v)
 }
 
 /* lane state of k_frame, packed into three words so that the kernel needs
- * few more registers than the separate launches (88-89 against 78-79, 5
- * waves per SIMD): gp = the ray's batch pixel; k = the camera ray's work
+ * few more registers than the separate launches (96 and a spill outside the
+ * step against 91-95, 5 waves per SIMD; 4 waves without it: 3.39 against
+ * 3.27 ms on a 1080p frame of 90M points): gp = the ray's batch pixel; k = the camera ray's work
  * item, or the shadow ray's slot; tag = kind bits, the sprite slot of a
  * sprite trace, and the lights still deferred to this lane (bits 8..15) */
 constexpr uint32_t kTagShadow = 0x80000000u; /* the lane's ray is a shadow ray */

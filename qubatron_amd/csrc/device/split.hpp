@@ -96,6 +96,7 @@ __device__ __forceinline__ void drain(const SceneDev& s, Ray& r, const Stack& st
                 seg = trace_step<CMP, DUAL, SEM, GRID>(s, r, st, t);
                 if (seg != ST_CONT) break;
             }
+            if (count_steps<CMP, DUAL>(s, t, kBurst) && seg == ST_CONT) seg = ST_ABORT;
         }
         /* the lowest hit of every ray (an aborted segment ends its ray like a
          * hit), then its lowest unfinished key */
@@ -149,13 +150,12 @@ __device__ __forceinline__ void drain(const SceneDev& s, Ray& r, const Stack& st
             const int  v     = takes ? (int) mail[irank] : lane;
             const int  l0    = below != 0u ? __ffs((int) below) - 1 : 0; /* the giver's shallowest pending level */
             const int  lv    = __shfl(l0, v, 64);
+            const uint32_t pv = __shfl(t.pend, v, 64);
             uint32_t   cut   = (b - a) >> 3; /* the upper end goes with the entries: the giver shares more often */
             cut              = b - (cut ? cut : 1u);
             r.px = __shfl(r.px, v, 64), r.py = __shfl(r.py, v, 64), r.pz = __shfl(r.pz, v, 64);
             r.dx = __shfl(r.dx, v, 64), r.dy = __shfl(r.dy, v, 64), r.dz = __shfl(r.dz, v, 64);
             r.ix = __shfl(r.ix, v, 64), r.iy = __shfl(r.iy, v, 64), r.iz = __shfl(r.iz, v, 64);
-            t.start.x = __shfl(t.start.x, v, 64), t.start.y = __shfl(t.start.y, v, 64);
-            t.start.z = __shfl(t.start.z, v, 64), t.start.w = __shfl(t.start.w, v, 64);
             t.level   = __shfl(t.level, v, 64);
             t.ix = __shfl(t.ix, v, 64), t.iy = __shfl(t.iy, v, 64), t.iz = __shfl(t.iz, v, 64);
             t.it                = __shfl(t.it, v, 64);
@@ -173,7 +173,7 @@ __device__ __forceinline__ void drain(const SceneDev& s, Ray& r, const Stack& st
                 const int sh = t.level - (lv + 1);
                 t.ix >>= sh, t.iy >>= sh, t.iz >>= sh;
                 t.level = lv + 1;
-                t.pend  = 1u << lv;
+                t.pend  = (pv & kRayBits) | 1u << lv;
                 seg     = trace_pop<CMP, DUAL, SEM, GRID>(s, r, st, t);
             } else if (gives && grank < pairs) {
                 b = cut;
@@ -277,24 +277,32 @@ __device__ __forceinline__ int keep_active(const Refill& rf, unsigned refill)
     return rf.left > 0 ? 65 - (int) refill : 1; /* refill when idle lanes >= refill */
 }
 
+constexpr int kRunSteps = 4096; /* most steps between two looks at the iteration cap */
+
 template <bool CMP, bool DUAL, int SEM, bool GRID>
 __device__ __forceinline__ void step_run(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t, bool& active,
                                          int keep, int& fin)
 {
+    int steps = 0; /* of the wave in this call: uniform */
     for (;;) {
         const int stt = trace_step<CMP, DUAL, SEM, GRID>(s, r, st, t);
+        steps++;
         if (stt != ST_CONT) {
             fin    = stt;
             active = false;
             break;
         }
-        if (__popcll(__ballot(1)) < keep) break;
+        if (__popcll(__ballot(1)) < keep || steps == kRunSteps) break;
+    }
+    if (count_steps<CMP, DUAL>(s, t, steps) && active) {
+        fin    = ST_ABORT;
+        active = false;
     }
 }
 
 /* Blocks of a persistent traversal launch over at most `items` rays: all
- * that are resident (5 or 6 waves per SIMD for the traversal kernels: VGPRs and
- * LDS stacks), at most one lane per ray, but not fewer than
+ * that are resident (5 waves per SIMD for the traversal kernels: VGPRs and LDS
+ * stacks), at most one lane per ray, but not fewer than
  * kSpreadWavesPerSimd waves per SIMD: those then take fewer rays each
  * (Refill::share), down to one. A wave alone on its SIMD steps at its own
  * latency, so a second one is nearly free, and the lanes without a ray take

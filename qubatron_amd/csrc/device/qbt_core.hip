@@ -1026,7 +1026,7 @@ int qbt_ctx::scene_for(const float basecube[4], int maxlevel, SceneDev& s, bool&
                 tb.cmp_stale = false;
             }
         }
-        cmp = tree[0].cmp.ok && (!dual || tree[1].cmp.ok);
+        cmp = tree[0].cmp.ok && (!dual || (tree[1].cmp.ok && tree[1].cmp.n < kDualRecords));
     }
     memset(&s, 0, sizeof(s));
     for (int t = 0; t < 2; t++) {

@@ -280,13 +280,8 @@ __device__ __forceinline__ unsigned exist_mask(int4 lo, int4 hi)
            (hi.x > 0 ? 16u : 0u) | (hi.y > 0 ? 32u : 0u) | (hi.z > 0 ? 64u : 0u) | (hi.w > 0 ? 128u : 0u);
 }
 
-/* The child block of one node in either layout: the 8 child indices of the
- * direct layout (two int4), or the compact {first child, mask} record. */
-template <bool CMP>
-struct Block;
-
-template <>
-struct Block<false> {
+/* The child block of one node in the direct layout: 8 child indices. */
+struct Block {
     int4 lo, hi;
     __device__ __forceinline__ void clear() { lo = hi = make_int4(0, 0, 0, 0); }
     __device__ __forceinline__ void load(const TreeDev& t, int i)
@@ -304,17 +299,6 @@ struct Block<false> {
  * o is record x + (the number of alloc bits below o). Live is a subset of
  * alloc; they differ only where an in-place range update zeroed a slot and
  * left its record in the block. */
-template <>
-struct Block<true> {
-    uint2 r;
-    __device__ __forceinline__ void     clear() { r = make_uint2(0u, 0u); }
-    __device__ __forceinline__ void     load(const TreeDev& t, int i) { r = t.rec[i]; }
-    __device__ __forceinline__ unsigned mask() const { return r.y & 0xFFu; }
-    __device__ __forceinline__ int      child(int o) const
-    {
-        return ((r.y >> o) & 1u) ? (int) (r.x + (uint32_t) __popc((r.y >> 8) & ((1u << o) - 1u))) : 0;
-    }
-};
 
 /* The particle shader addresses slot k of node i as texel
  * (3 i mod 8192 + k / 4, 3 i / 8192) (particle_vsh.c:110-119): the texel
@@ -327,27 +311,21 @@ struct Block<true> {
 __device__ __forceinline__ bool particle_hi_lost(int i) { return ((uint32_t) i * 3u) % 8192u == 8191u; }
 __device__ __forceinline__ bool particle_model_lost(int i) { return ((uint32_t) i * 3u) % 8192u >= 8190u; }
 
-/* the child block of node i as the semantics SEM reads it (direct layout) */
+/* the child block of node i as the semantics SEM reads it */
 template <int SEM>
-__device__ __forceinline__ void load_block(Block<false>& b, const TreeDev& t, int i)
+__device__ __forceinline__ void load_block(Block& b, const TreeDev& t, int i)
 {
     b.load(t, i);
     if (SEM == kSemParticle && particle_hi_lost(i)) b.hi = make_int4(0, 0, 0, 0);
 }
-template <int SEM>
-__device__ __forceinline__ void load_block(Block<true>& b, const TreeDev& t, int i)
-{
-    static_assert(SEM != kSemParticle, "the particle semantics addresses reference node indices: direct layout");
-    b.load(t, i);
-}
 
 /* slot k (< 8) of node i at `level` (oct_from_octets_for_index,
  * octree_fsh.c:127-136): 0 for index 0 below the root. */
-template <bool CMP, int SEM = kSemShader>
+template <int SEM>
 __device__ __forceinline__ int child_slot(const TreeDev& t, int i, int k, int level)
 {
     if (i == 0 && level > 0) return 0;
-    Block<CMP> b;
+    Block b;
     load_block<SEM>(b, t, i);
     return b.child(k);
 }
@@ -411,6 +389,10 @@ struct TraceState {
 };
 
 enum : int { ST_CONT = 2 };
+
+/* records a dynamic compact layout may have when both trees are walked
+ * (trace_step_c2's stack words) */
+constexpr uint32_t kDualRecords = 1u << 24;
 
 constexpr uint32_t kSlowRay   = 0x80000000u; /* in pend: the ray's quotients need plane_k's check */
 constexpr int      kFaceShift = 28;
@@ -682,7 +664,7 @@ __device__ __forceinline__ bool expand_general_position(const SceneDev& s, const
     return !bad;
 }
 
-/* Entry point of the child behind `plane` (1 x, 2 y, 4 z) of the node at
+/* Entry point of the child behind `plane` (1 x, 2 y, 3 or 4 z) of the node at
  * level j whose cell coordinates are (ix, iy, iz) >> sh, or, plane 0, the
  * root entry: midplane_cell's and root_entry's, the quotient unchecked where
  * the ray allows. On an exact grid the mid-plane's coordinate is one FMA:
@@ -812,12 +794,115 @@ __device__ __forceinline__ int trace_pop_c1(const SceneDev& s, const Ray& r, con
     return t.level == s.maxlevel ? ST_HIT : ST_CONT;
 }
 
+/*
+ * Both trees on their compact layouts, in the manner of trace_step_c1: one
+ * path for descending and backtracking lanes, and backtracking never re-reads
+ * a node. The words of a level:
+ *   pw word  up to three pending entries, 8 bits each, the next one lowest
+ *            (0: none): octet | plane << 3 as above | the child exists in the
+ *            static tree << 6, in the dynamic one << 7; bits 24-31 the static
+ *            node's slots
+ *   ns word  the static node's first child (30 bits) | the plane of the entry
+ *            being visited << 30 (1 x, 2 y, 3 z, 0 the node's entry point)
+ *   nd word  the dynamic node's first child (24 bits) | its slots << 24
+ * so the dynamic layout has fewer than kDualRecords records; beyond that both
+ * trees are walked on the direct layout. A node index is 0 where the path has
+ * left its tree. Against the direct layout's step on compact records (separate
+ * descend and backtrack paths, records read again on a backtrack), 720p over
+ * 5M static and 150k dynamic points: k_primary 633 -> 597 us, 719 -> 668 and
+ * 202 -> 210 (three poses), k_shadow 292 -> 261, 403 -> 357, 96 -> 92.
+ */
+/* the plane of an entry's bits 3-5 (one-hot) as a number: 1 x, 2 y, 3 z */
+__device__ __forceinline__ uint32_t plane_code(uint32_t e)
+{
+    const uint32_t p = (e >> 3) & 7u;
+    return p - (p >> 2);
+}
+
+/* the second half of a step: entry e (8 bits) of level lv becomes the current
+ * one; an, pw and ad are that level's new words (an without the plane) */
+template <int SEM, bool GRID>
+__device__ __forceinline__ int enter_c2(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t, bool keep,
+                                        int lv, uint32_t e, uint32_t pw, uint32_t an, uint32_t ad)
+{
+    const int at = st.at(lv), level = t.level;
+    int       j = lv, plane = (int) plane_code(e);
+    st.pw[at] = pw;
+    st.ns[at] = (int) (an | (uint32_t) plane << 30);
+    st.nd[at] = (int) ad;
+    if (!keep) {
+        while (plane == 0 && j > 0) {
+            j--;
+            plane = (int) ((uint32_t) st.ns[st.at(j)] >> 30);
+        }
+    }
+    if (!keep || plane != 0) t.entry = plane_entry<SEM, GRID>(s, r, t, plane, j, level - j);
+    const int      sh = level - lv, o = (int) (e & 7u);
+    const uint32_t cs = an + (uint32_t) __popc(__builtin_amdgcn_ubfe(pw, 24u, (uint32_t) o));
+    const uint32_t cd = (ad & 0xFFFFFFu) + (uint32_t) __popc(__builtin_amdgcn_ubfe(ad, 24u, (uint32_t) o));
+    t.ns    = (e & 64u) ? (int) cs : 0;
+    t.nd    = (e & 128u) ? (int) cd : 0;
+    t.ix    = ((t.ix >> sh) << 1) | (o & 1);
+    t.iy    = ((t.iy >> sh) << 1) | ((o >> 1) & 1);
+    t.iz    = ((t.iz >> sh) << 1) | (o >> 2);
+    t.level = lv + 1;
+    return t.level == s.maxlevel ? ST_HIT : ST_CONT;
+}
+
+template <int SEM, bool GRID>
+__device__ __forceinline__ int trace_step_c2(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
+{
+    const int      level = t.level;
+    const uint2    rs = s.stat.rec[(uint32_t) t.ns], rd = s.dyn.rec[(uint32_t) t.nd]; /* the root where there is none */
+    const bool     hs = t.ns != 0 || level == 0, hd = t.nd != 0 || level == 0;
+    const uint32_t ms = hs ? rs.y & 0xFFu : 0u, md = hd ? rd.y & 0xFFu : 0u;
+    t.exps += (hs ? 1u : 0u) + (hd ? 1u : 0u);
+    uint32_t word = 0;
+    int      n    = 0;
+    if (!GRID || !expand_general_position(s, r, t, ms | md, word, n)) word = expand_any<SEM, GRID>(s, r, t, ms | md, n);
+
+    const bool     desc  = n > 0;
+    const uint32_t below = t.pend & ((1u << level) - 1u);
+    if (!desc && below == 0u) return ST_MISS;
+    const int      lv  = desc ? level : 31 - __clz((int) below);
+    const int      at  = st.at(lv);
+    const uint32_t pwv = st.pw[at], an = (uint32_t) st.ns[at], ad = (uint32_t) st.nd[at];
+    /* the entries with their trees; entries past the n-th are dropped */
+    const uint32_t mm = ms << 6 | md << 15; /* bit 6 + o, 15 + o */
+    auto tree_bits = [&](uint32_t e) -> uint32_t {
+        const uint32_t b = mm >> (e & 7u);
+        return (b & 64u) | ((b >> 8) & 128u);
+    };
+    const uint32_t e0 = word & 63u, e1 = (word >> 6) & 63u, e2 = (word >> 12) & 63u, e3 = (word >> 18) & 63u;
+    const uint32_t p  = (e1 | tree_bits(e1)) | (e2 | tree_bits(e2)) << 8 | (e3 | tree_bits(e3)) << 16;
+    const uint32_t pn = p & ((1u << ((uint32_t) (8 * n - 8) & 31u)) - 1u);
+    const uint32_t e  = desc ? e0 | tree_bits(e0) : pwv & 0xFFu;
+    const uint32_t w  = desc ? pn | (rs.y >> 8) << 24 : ((pwv & 0xFFFFFFu) >> 8) | (pwv & 0xFF000000u);
+    /* descending: bit `level` set when more than one entry was kept;
+     * backtracking: bit lv cleared when this was its level's last one */
+    const uint32_t more = (w & 0xFFFFFFu) != 0u ? 1u : 0u;
+    t.pend = desc ? t.pend | more << level : t.pend ^ ((1u ^ more) << lv);
+    return enter_c2<SEM, GRID>(s, r, st, t, desc, lv, e, w, desc ? rs.x : an & 0x3FFFFFFFu,
+                               desc ? (rd.x & 0xFFFFFFu) | (rd.y >> 8) << 24 : ad);
+}
+
+/* the backtrack half of trace_step_c2 (as trace_pop_c1) */
+template <int SEM, bool GRID>
+__device__ __forceinline__ int trace_pop_c2(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
+{
+    const uint32_t below = t.pend & ((1u << t.level) - 1u);
+    const int      lv = 31 - __clz((int) below), at = st.at(lv);
+    const uint32_t pwv = st.pw[at], an = (uint32_t) st.ns[at], ad = (uint32_t) st.nd[at];
+    const uint32_t w   = ((pwv & 0xFFFFFFu) >> 8) | (pwv & 0xFF000000u);
+    t.pend ^= ((w & 0xFFFFFFu) != 0u ? 0u : 1u) << lv;
+    return enter_c2<SEM, GRID>(s, r, st, t, false, lv, pwv & 0xFFu, w, an & 0x3FFFFFFFu, ad);
+}
+
 /* backtrack (octree_fsh.c:368-375) and pop the next pending entry of the
  * deepest level below t.level that has one; ST_MISS where none has */
-template <bool CMP, bool DUAL, int SEM, bool GRID>
-__device__ __forceinline__ int trace_pop(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
+template <bool DUAL, int SEM, bool GRID>
+__device__ __forceinline__ int trace_pop_direct(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
 {
-    if constexpr (CMP && !DUAL) return trace_pop_c1<SEM, GRID>(s, r, st, t);
     /* the deepest level with a pending entry, from the per-lane mask (bit l
      * set while level l has one; the levels between have none) */
     const int      level = t.level;
@@ -837,8 +922,8 @@ __device__ __forceinline__ int trace_pop(const SceneDev& s, const Ray& r, const 
     } else {
         isp = midplane_cell<SEM, GRID>(s, r, src, lv, ix, iy, iz, 0);
     }
-    t.ns    = child_slot<CMP, SEM>(s.stat, st.ns[lv * st.stride], o, lv);
-    t.nd    = DUAL ? child_slot<CMP>(s.dyn, st.nd[lv * st.stride], o, lv) : 0;
+    t.ns    = child_slot<SEM>(s.stat, st.ns[lv * st.stride], o, lv);
+    t.nd    = DUAL ? child_slot<kSemShader>(s.dyn, st.nd[lv * st.stride], o, lv) : 0;
     t.ix    = (ix << 1) | (o & 1);
     t.iy    = (iy << 1) | ((o >> 1) & 1);
     t.iz    = (iz << 1) | (o >> 2);
@@ -847,21 +932,15 @@ __device__ __forceinline__ int trace_pop(const SceneDev& s, const Ray& r, const 
     return t.level == s.maxlevel ? ST_HIT : ST_CONT;
 }
 
-/*
- * One step: expand the node just entered and descend into its nearest
- * pending child, or backtrack and descend into the next pending child of an
- * ancestor. Returns ST_CONT, ST_HIT (t.level == maxlevel; the leaf is
- * t.ns / t.nd with entry point t.entry), ST_MISS or ST_ABORT.
- */
-template <bool CMP, bool DUAL, int SEM, bool GRID>
-__device__ __forceinline__ int trace_step(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
+/* The step on the direct layout, one tree or both; counts itself in t.it. */
+template <bool DUAL, int SEM, bool GRID>
+__device__ __forceinline__ int trace_step_direct(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
 {
-    if constexpr (CMP && !DUAL) return trace_step_c1<SEM, GRID>(s, r, st, t);
     if (++t.it > s.iter_cap) return ST_ABORT;
     const int level = t.level;
 
     /* ---- expansion of the node just entered (octree_fsh.c:251-330) ---- */
-    Block<CMP> sb, db;
+    Block sb, db;
     sb.clear();
     db.clear();
     if (t.ns != 0 || level == 0) {
@@ -880,7 +959,7 @@ __device__ __forceinline__ int trace_step(const SceneDev& s, const Ray& r, const
         cube_at<GRID>(s, level, t.ix, t.iy, t.iz, tx, ty, tz, tw);
         cube_mid<GRID>(tx, ty, tz, tw, bxx, byy, bzz, hx, hy, hz);
 
-        /* candidates as (t, key) pairs, as in trace_step_c1 */
+        /* candidates as (t, key) pairs, as in expand_any */
         const float  qnan = __builtin_nanf("");
         const float4 az   = plane_z<SEM>(hz, r);
         const float4 ax   = plane_x<SEM>(hx, r);
@@ -942,7 +1021,31 @@ __device__ __forceinline__ int trace_step(const SceneDev& s, const Ray& r, const
         }
     }
 
-    return trace_pop<CMP, DUAL, SEM, GRID>(s, r, st, t);
+    return trace_pop_direct<DUAL, SEM, GRID>(s, r, st, t);
+}
+
+/*
+ * One step: expand the node just entered and descend into its nearest
+ * pending child, or backtrack and descend into the next pending child of an
+ * ancestor. Returns ST_CONT, ST_HIT (t.level == maxlevel; the leaf is
+ * t.ns / t.nd with entry point t.entry), ST_MISS or ST_ABORT.
+ */
+template <bool CMP, bool DUAL, int SEM, bool GRID>
+__device__ __forceinline__ int trace_step(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
+{
+    if constexpr (CMP && DUAL) return trace_step_c2<SEM, GRID>(s, r, st, t);
+    else if constexpr (CMP) return trace_step_c1<SEM, GRID>(s, r, st, t);
+    else return trace_step_direct<DUAL, SEM, GRID>(s, r, st, t);
+}
+
+/* backtrack only: the next pending entry of the deepest level below t.level
+ * that has one */
+template <bool CMP, bool DUAL, int SEM, bool GRID>
+__device__ __forceinline__ int trace_pop(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
+{
+    if constexpr (CMP && DUAL) return trace_pop_c2<SEM, GRID>(s, r, st, t);
+    else if constexpr (CMP) return trace_pop_c1<SEM, GRID>(s, r, st, t);
+    else return trace_pop_direct<DUAL, SEM, GRID>(s, r, st, t);
 }
 
 /* Counts the steps just taken (steps that do not count themselves) and
@@ -950,7 +1053,7 @@ __device__ __forceinline__ int trace_step(const SceneDev& s, const Ray& r, const
 template <bool CMP, bool DUAL>
 __device__ __forceinline__ bool count_steps(const SceneDev& s, TraceState& t, int steps)
 {
-    if constexpr (CMP && !DUAL) {
+    if constexpr (CMP) {
         t.it += steps;
         return t.it > s.iter_cap;
     }

@@ -116,9 +116,9 @@ __device__ __forceinline__ uint32_t* wave_mail(uint32_t* lds, int L)
  * b.sprite), then nitems pixel items.
  *
  * Bound by the issue of the traversal step's vector instructions and, towards
- * the end, by the latency of a lone wave's step. Five waves per SIMD (91
- * VGPRs): at six the slow paths spill, and 2.07M short rays take 352 us
- * against 328 (long ones, 8.3M of a 2160p frame, 6.32 against 6.49 ms). */
+ * the end, by the latency of a lone wave's step. Five waves per SIMD (87
+ * VGPRs): at six the slow paths spill, and 2.07M short rays take 313 us
+ * against 304 (long ones, 8.3M of a 2160p frame, 5.32 against 5.51 ms). */
 template <bool CMP, bool DUAL, bool GRID, bool COUNT, bool GSTK>
 __global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, PrimOut o, uint32_t nitems, uint32_t nspr,
                                                  int nl, int strip, int* __restrict__ sprite, unsigned* __restrict__ q,
@@ -483,9 +483,10 @@ __global__ void k_oct_scan(const unsigned* __restrict__ cnt, unsigned* __restric
  * (lexp: per light, counting renders), so the frame does not depend on the
  * order in which rays end (the sample collector applies the same rule).
  *
- * Five waves per SIMD (95 VGPRs) against six, which spill: 536 against 560
- * us on the shadow rays of a 1080p frame of 10M points, 1.82 against 1.87 ms
- * on a batch of 12 views; 8.58 against 8.49 ms on a 2160p frame of 30M. */
+ * Five waves per SIMD (91 VGPRs); six spill, and with a longer step (95
+ * VGPRs) took 560 against 536 us on the shadow rays of a 1080p frame of 10M
+ * points, 1.87 against 1.82 ms on a batch of 12 views, 8.49 against 8.58 ms
+ * on a 2160p frame of 30M. */
 template <bool CMP, bool DUAL, bool GRID, bool COUNT, bool GSTK>
 __global__ void __launch_bounds__(256, 5)
     k_shadow(SceneDev s, LightsDev L, const uint32_t* __restrict__ lists,

@@ -55,15 +55,6 @@ enum : int {
 #define QBT_OPAQUE(x) asm volatile("" : "+v"(x))
 #endif
 
-/* The same on a wave-uniform value: it stays in a scalar register until it
- * is used (the compiler would otherwise copy loop-invariant scalars that a
- * select needs to vector registers outside the loop, and spill them). */
-#ifdef __HIP__
-#define QBT_OPAQUE_S(x) asm volatile("" : "+s"(x))
-#else
-#define QBT_OPAQUE_S(x) ((void) 0)
-#endif
-
 enum TraceStatus : int { ST_MISS = 0, ST_HIT = 1, ST_DISCARD = -1, ST_ABORT = -2 };
 
 struct TreeDev {
@@ -350,16 +341,16 @@ struct Stack {
 };
 
 /* Root entry point of a ray, recomputed from the face that trace_begin found
- * (the same operations, so the same bits): 0 the ray starts in the cube, 1, 2
- * the z planes at base and far end, 3, 4 x, 5, 6 y. A face is three bits
- * where the point is four registers. */
+ * (the same operations, so the same bits): its plane, 1 x, 2 y, 3 z, 0 the ray
+ * starts in the cube, and 4 for the far one. A face is three bits where the
+ * point is four registers. */
 template <int SEM>
 __device__ __forceinline__ float4 root_entry(const SceneDev& s, const Ray& r, int face)
 {
     if (face == 0) return make_float4(r.px, r.py, r.pz, 0.0f);
-    const int   k = face <= 2 ? 2 : (face <= 4 ? 0 : 1);
+    const int   k = (face & 3) - 1;
     const float b = axis3(k, s.bx, s.by, s.bz), f = k == 0 ? b + s.bw : b - s.bw;
-    return plane_k<SEM>(k, (face & 1) ? b : f, r);
+    return plane_k<SEM>(k, (face & 4) ? f : b, r);
 }
 
 /* Entry point of the node at `level` on the current path (level >= 1 uses
@@ -448,15 +439,15 @@ __device__ __forceinline__ int trace_begin(const SceneDev& s, Ray& r, TraceState
         hitc++;                                  \
     }
         a = plane_z<SEM>(tz, r);
-        QBT_CONSIDER(1, tx < a.x && a.x <= rx && ty > a.y && a.y >= ry)
+        QBT_CONSIDER(3, tx < a.x && a.x <= rx && ty > a.y && a.y >= ry)
         a = plane_z<SEM>(rz, r);
-        QBT_CONSIDER(2, tx < a.x && a.x <= rx && ty > a.y && a.y >= ry)
+        QBT_CONSIDER(7, tx < a.x && a.x <= rx && ty > a.y && a.y >= ry)
         a = plane_x<SEM>(tx, r);
-        QBT_CONSIDER(3, ty > a.y && a.y >= ry && tz > a.z && a.z >= rz)
+        QBT_CONSIDER(1, ty > a.y && a.y >= ry && tz > a.z && a.z >= rz)
         a = plane_x<SEM>(rx, r);
-        QBT_CONSIDER(4, ty > a.y && a.y >= ry && tz > a.z && a.z >= rz)
+        QBT_CONSIDER(5, ty > a.y && a.y >= ry && tz > a.z && a.z >= rz)
         a = plane_y<SEM>(ty, r);
-        QBT_CONSIDER(5, tx < a.x && a.x <= rx && tz > a.z && a.z >= rz)
+        QBT_CONSIDER(2, tx < a.x && a.x <= rx && tz > a.z && a.z >= rz)
         a = plane_y<SEM>(ry, r);
         QBT_CONSIDER(6, tx < a.x && a.x <= rx && tz > a.z && a.z >= rz)
 #undef QBT_CONSIDER
@@ -500,6 +491,9 @@ __device__ __forceinline__ float4 pick_entry(int src, float4 e, float4 z, float4
     if (src == 3) r = y;
     return r;
 }
+
+/* the highest set bit of m, which is not 0 */
+__device__ __forceinline__ int top_bit(uint32_t m) { return 31 - __builtin_clz(m); }
 
 /* bit o of m (one bit-field extract) */
 __device__ __forceinline__ bool bit_of(uint32_t m, int o) { return __builtin_amdgcn_ubfe(m, (uint32_t) o, 1u) != 0u; }
@@ -610,11 +604,14 @@ __device__ __forceinline__ uint32_t expand_any(const SceneDev& s, const Ray& r, 
  * crossing flips the bit of its own plane and nothing else (the reference's
  * octet by coordinates, and its tie-flipped octet where that equals the one
  * before, come to the same), and the sort needs the keys alone. false where
- * any of this does not hold: the caller takes expand_any. The step's main
- * block is 135 vector instructions against 173 and has one rare branch
- * instead of four; with plane_entry and the 6-bit entries, k_primary +
- * k_shadow of a 2160p frame of 30M points 15.38 -> 15.07 ms (long rays, seed
- * 6) and 4.86 -> 4.77 ms (short ones), 200k free rays 238 -> 207 us. */
+ * any of this does not hold: the caller takes expand_any. The traversal of
+ * large frames is bound by the issue of vector instructions (about 160 node
+ * expansions per ns), so the step is written for their number: 118 to here
+ * against 173 of expand_any and the checks of its quotients, one rare branch
+ * instead of four. k_primary + k_shadow of a 2160p frame of 30M points took
+ * 15.38 ms with expand_any alone, 15.07 with a first form of this (the keys
+ * from the hits' coordinates, 135 instructions; 62 in plane_entry), 12.83 now
+ * (44 in plane_entry); 200k free rays 238, 209 and 190 us. */
 __device__ __forceinline__ bool expand_general_position(const SceneDev& s, const Ray& r, const TraceState& t,
                                                         uint32_t mask, uint32_t& word, int& n)
 {
@@ -637,21 +634,23 @@ __device__ __forceinline__ bool expand_general_position(const SceneDev& s, const
     /* the order of the hits; ties as the network leaves them: z, x, y, but
      * for z and x level behind y */
     const bool xbz = wx < wz, ybz = wy < wz, ybx = wy < wx;
-    bool       bad = (t.pend & kSlowRay) != 0u;
-    bad |= fminf(fminf(wz, wx), wy) < t.entry.w;
-    bad |= (zx == hx) | (zy == hy) | (yx == hx) | ((wx == wz) & vz & ybx);
-    bad |= vz & ((gzx ^ ex ^ xbz) | (gzy ^ ey ^ ybz));
-    bad |= vx & ((gxz ^ ez ^ !xbz) | (gxy ^ ey ^ ybx));
-    bad |= vy & ((gyz ^ ez ^ !ybz) | (gyx ^ ex ^ !ybx));
-    /* keys: entries, or an octet that the mask does not have */
+    /* (logical operators: as numbers the conditions would go through vector
+     * registers) */
+    const bool slow = (t.pend & kSlowRay) != 0u, early = fminf(fminf(wz, wx), wy) < t.entry.w;
+    const bool tie = (zx == hx) || (zy == hy) || (yx == hx), level = (wx == wz) && vz && ybx;
+    const bool mz = vz && ((gzx != (ex != xbz)) || (gzy != (ey != ybz)));
+    const bool mx = vx && ((gxz != (ez != !xbz)) || (gxy != (ey != ybx)));
+    const bool my = vy && ((gyz != (ez != !ybz)) || (gyx != (ex != !ybx)));
+    const bool bad = slow || early || tie || level || mz || mx || my;
+    /* the crossings in order, c = plane << 3 | plane, or 24 for none (it sorts
+     * last): each flips its bit of the octet before and gives its entry;
+     * behind the last one an octet that the mask does not have */
     const uint32_t o0 = (ex ? 1u : 0u) | (ey ? 2u : 0u) | (ez ? 4u : 0u);
-    const uint32_t no = ~o0;
-    const uint32_t kz = vz ? (gzx ? 1u : 0u) | (gzy ? 2u : 0u) | (no & 4u) | 32u : 24u;
-    const uint32_t kx = vx ? (no & 1u) | (gxy ? 2u : 0u) | (gxz ? 4u : 0u) | 8u : 24u;
-    const uint32_t ky = vy ? (gyx ? 1u : 0u) | (no & 2u) | (gyz ? 4u : 0u) | 16u : 24u;
-    const uint32_t k1 = xbz ? (ybx ? ky : kx) : (ybz ? ky : kz);
-    const uint32_t k3 = xbz ? (ybz ? kz : ky) : (ybx ? kx : ky);
-    const uint32_t k2 = kz ^ kx ^ ky ^ k1 ^ k3;
+    const uint32_t cz = vz ? 36u : 24u, cx = vx ? 9u : 24u, cy = vy ? 18u : 24u;
+    const uint32_t c1 = xbz ? (ybx ? cy : cx) : (ybz ? cy : cz);
+    const uint32_t c3 = xbz ? (ybz ? cz : cy) : (ybx ? cx : cy);
+    const uint32_t c2 = cz ^ cx ^ cy ^ c1 ^ c3;
+    const uint32_t k1 = o0 ^ c1, k2 = (k1 & 7u) ^ c2, k3 = (k2 & 7u) ^ c3;
     /* the live mask once per plane: an entry's low five bits (octet and x, y
      * plane bits) are its bit, 24..31 (no candidate) are zero */
     const uint32_t m3 = mask | mask << 8 | mask << 16;
@@ -678,15 +677,12 @@ __device__ __forceinline__ float4 plane_entry(const SceneDev& s, const Ray& r, c
         return plane == 0 ? root_entry<SEM>(s, r, root_face(t))
                           : midplane_cell<SEM, GRID>(s, r, plane == 1 ? 2 : (plane == 2 ? 3 : 1), j, t.ix, t.iy, t.iz, sh);
     const bool root = plane == 0;
-    const int  f = root_face(t), ax = root ? (f + 1) >> 1 : plane; /* root: 1 z, 2 x, 3 y, 0 inside */
-    const bool px = root ? ax == 2 : plane == 1, py = root ? ax == 3 : plane == 2, in = root && f == 0;
+    const int  f = root_face(t), at = root ? f & 3 : plane;
+    const bool px = at == 1, py = at == 2, in = at == 0;
     const int  i = sel(px, t.ix, sel(py, t.iy, t.iz)) >> sh;
-    const int  m = root ? ((f & 1) ? 0 : 2) : 2 * i + 1;
+    const int  m = root ? (f >> 1) & 2 : 2 * i + 1;
     const float h = ldexpf(s.bw, -1 - j);
-    float bx = s.bx, by = s.by, bz = s.bz;
-    QBT_OPAQUE_S(bx);
-    QBT_OPAQUE_S(by);
-    QBT_OPAQUE_S(bz);
+    const float bx = s.bx, by = s.by, bz = s.bz;
     const float c = __builtin_fmaf((float) m, px ? h : -h, px ? bx : (py ? by : bz));
     /* values, not the ray's members: a select between members is a load from
      * a selected address, and the ray then lives in memory */
@@ -728,19 +724,18 @@ __device__ __forceinline__ int trace_step_c1(const SceneDev& s, const Ray& r, co
     if (!desc && below == 0u) return ST_MISS;
     /* the deepest level with a pending entry, from the per-lane mask (levels
      * between it and this one have none: no loop over them) */
-    const int      lv  = desc ? level : 31 - __clz((int) below);
+    const int      lv  = desc ? level : top_bit(below);
     const int      at  = st.at(lv);
     const uint32_t an  = (uint32_t) st.ns[at];
     const uint32_t pwv = st.pw[at];
     /* backtracking: the next entry of level lv becomes the current one */
     const uint32_t w   = desc ? word : ((pwv & 0xFFFFFFu) >> 6) | (pwv & 0xFF000000u);
+    const uint32_t nw = desc ? rec.x | (uint32_t) (n - 1) << 30 : an - (1u << 30);
     st.pw[at] = w;
-    st.ns[at] = (int) (desc ? rec.x | (uint32_t) (n - 1) << 30 : an - (1u << 30));
-    /* descending: bit `level` set when more than one entry was kept;
-     * backtracking: bit lv cleared when this was the level's last pending
-     * entry (count field 1: bit 31 of the node word clear) */
-    t.pend = desc ? t.pend | (n > 1 ? 1u : 0u) << level : t.pend ^ ((1u << lv) & ~(uint32_t) ((int) an >> 31));
-    const uint32_t a = desc ? rec.x : an & 0x3FFFFFFFu;
+    st.ns[at] = (int) nw;
+    /* bit lv: whether the level still has a pending entry */
+    t.pend = (t.pend & ~(1u << lv)) | (nw >= 1u << 30 ? 1u << lv : 0u);
+    const uint32_t a = nw & 0x3FFFFFFFu;
     /* Its entry point. Plane 0 (the node's own entry point): a descending
      * lane keeps its entry; a backtracking one takes the mid-plane hit of the
      * nearest node on the path entered through a mid-plane, else the root
@@ -778,7 +773,7 @@ __device__ __forceinline__ int trace_pop_c1(const SceneDev& s, const Ray& r, con
     const uint32_t w     = ((pwv & 0xFFFFFFu) >> 6) | (pwv & 0xFF000000u);
     st.pw[at] = w;
     st.ns[at] = (int) (an - (1u << 30));
-    t.pend ^= (1u << lv) & ~(uint32_t) ((int) an >> 31);
+    t.pend ^= an - (1u << 30) >= 1u << 30 ? 0u : 1u << lv;
     int j = lv, plane = (int) ((w >> 3) & 7u);
     while (plane == 0 && j > 0) {
         j--;
@@ -809,8 +804,8 @@ __device__ __forceinline__ int trace_pop_c1(const SceneDev& s, const Ray& r, con
  * trees are walked on the direct layout. A node index is 0 where the path has
  * left its tree. Against the direct layout's step on compact records (separate
  * descend and backtrack paths, records read again on a backtrack), 720p over
- * 5M static and 150k dynamic points: k_primary 633 -> 597 us, 719 -> 668 and
- * 202 -> 210 (three poses), k_shadow 292 -> 261, 403 -> 357, 96 -> 92.
+ * 5M static and 150k dynamic points: k_primary 633 -> 548 us, 719 -> 603 and
+ * 202 -> 200 (three poses), k_shadow 292 -> 247, 403 -> 342, 96 -> 88.
  */
 /* the plane of an entry's bits 3-5 (one-hot) as a number: 1 x, 2 y, 3 z */
 __device__ __forceinline__ uint32_t plane_code(uint32_t e)
@@ -864,7 +859,7 @@ __device__ __forceinline__ int trace_step_c2(const SceneDev& s, const Ray& r, co
     const bool     desc  = n > 0;
     const uint32_t below = t.pend & ((1u << level) - 1u);
     if (!desc && below == 0u) return ST_MISS;
-    const int      lv  = desc ? level : 31 - __clz((int) below);
+    const int      lv  = desc ? level : top_bit(below);
     const int      at  = st.at(lv);
     const uint32_t pwv = st.pw[at], an = (uint32_t) st.ns[at], ad = (uint32_t) st.nd[at];
     /* the entries with their trees; entries past the n-th are dropped */
@@ -878,10 +873,8 @@ __device__ __forceinline__ int trace_step_c2(const SceneDev& s, const Ray& r, co
     const uint32_t pn = p & ((1u << ((uint32_t) (8 * n - 8) & 31u)) - 1u);
     const uint32_t e  = desc ? e0 | tree_bits(e0) : pwv & 0xFFu;
     const uint32_t w  = desc ? pn | (rs.y >> 8) << 24 : ((pwv & 0xFFFFFFu) >> 8) | (pwv & 0xFF000000u);
-    /* descending: bit `level` set when more than one entry was kept;
-     * backtracking: bit lv cleared when this was its level's last one */
-    const uint32_t more = (w & 0xFFFFFFu) != 0u ? 1u : 0u;
-    t.pend = desc ? t.pend | more << level : t.pend ^ ((1u ^ more) << lv);
+    /* bit lv: whether the level still has a pending entry */
+    t.pend = (t.pend & ~(1u << lv)) | ((w & 0xFFFFFFu) != 0u ? 1u << lv : 0u);
     return enter_c2<SEM, GRID>(s, r, st, t, desc, lv, e, w, desc ? rs.x : an & 0x3FFFFFFFu,
                                desc ? (rd.x & 0xFFFFFFu) | (rd.y >> 8) << 24 : ad);
 }
@@ -891,7 +884,7 @@ template <int SEM, bool GRID>
 __device__ __forceinline__ int trace_pop_c2(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t)
 {
     const uint32_t below = t.pend & ((1u << t.level) - 1u);
-    const int      lv = 31 - __clz((int) below), at = st.at(lv);
+    const int      lv = top_bit(below), at = st.at(lv);
     const uint32_t pwv = st.pw[at], an = (uint32_t) st.ns[at], ad = (uint32_t) st.nd[at];
     const uint32_t w   = ((pwv & 0xFFFFFFu) >> 8) | (pwv & 0xFF000000u);
     t.pend ^= ((w & 0xFFFFFFu) != 0u ? 0u : 1u) << lv;

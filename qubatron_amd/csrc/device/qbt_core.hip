@@ -339,7 +339,7 @@ __device__ __forceinline__ unsigned trace_batch(const SceneDev& s, uint32_t n, G
     const int      lane = threadIdx.x & 63;
     uint32_t*      mail = lds + blockDim.x * (uint32_t) (s.maxlevel > 0 ? s.maxlevel : 1) * (DUAL ? 3u : 2u) +
                      (threadIdx.x & ~63u);
-    constexpr int  refill = 16;
+    constexpr unsigned refill = 16;
     bool           active = false;
     uint32_t       item   = 0;
     Ray            r      = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -358,7 +358,7 @@ __device__ __forceinline__ unsigned trace_batch(const SceneDev& s, uint32_t n, G
             fin = ST_CONT;
         }
         const uint64_t idle = __ballot(!active);
-        if (given || (rf.left > 0 && (__popcll(idle) >= refill || idle == ~0ull))) {
+        if (given || (rf.left > 0 && __popcll(idle) >= (int) refill)) {
             const uint32_t k = given ? first : rf.fetch(q, idle, lane);
             given            = false;
             if (k != UINT32_MAX) {
@@ -377,7 +377,7 @@ __device__ __forceinline__ unsigned trace_batch(const SceneDev& s, uint32_t n, G
             });
             break;
         }
-        if (active) step_run<CMP, DUAL, SEM, GRID>(s, r, st, t, active, keep_active(rf, refill), fin);
+        if (active) step_run<CMP, DUAL, SEM, GRID>(s, r, st, t, active, false, refill, fin);
     }
     return n_abort;
 }

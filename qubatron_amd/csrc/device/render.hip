@@ -195,13 +195,15 @@ __global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, Prim
     int      fin   = ST_CONT; /* status of a ray that ended and awaits its outputs */
     uint32_t first = UINT32_MAX;
     bool     given = rf.share(lane, first); /* few items: each wave its share, no queue */
+    bool     due   = false;
     for (;;) {
         if (fin != ST_CONT) { /* rays that ended since the last refill point, together */
             finish(fin);
             fin = ST_CONT;
         }
         const uint64_t idle = __ballot(!active);
-        if (given || (rf.left > 0 && (__popcll(idle) >= (int) refill || idle == ~0ull))) {
+        if (given || (rf.left > 0 && idle != 0ull && (due || __popcll(idle) >= (int) (refill & 255u)))) {
+            due = false;
             const uint32_t fetched = given ? first : rf.fetch(&q[Q_PRIM], idle, lane);
             given                  = false;
             if (fetched != UINT32_MAX) {
@@ -252,7 +254,8 @@ __global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, Prim
             if (rf.left <= 0) break;
             continue;
         }
-        if (active) step_run<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, keep_active(rf, refill), fin);
+        if (active) step_run<CMP, DUAL, kSemShader, GRID, true>(s, r, st, t, active, rf.left <= 0, refill, fin);
+        due = refill >= 256u; /* the step ended at the refill rule */
     }
     n_hit   = wave_sum(n_hit);
     n_abort = wave_sum(n_abort);
@@ -536,7 +539,7 @@ __global__ void __launch_bounds__(256, 5)
             fin = ST_CONT;
         }
         const uint64_t idle = __ballot(!active);
-        if (given || (rf.left > 0 && (__popcll(idle) >= (int) refill || idle == ~0ull))) {
+        if (given || (rf.left > 0 && __popcll(idle) >= (int) refill)) {
             const uint32_t k = given ? first : rf.fetch(&q[Q_SHADOW], idle, lane);
             given            = false;
             if (k != UINT32_MAX) {
@@ -587,7 +590,7 @@ __global__ void __launch_bounds__(256, 5)
             if (rf.left <= 0) break;
             continue;
         }
-        if (active) step_run<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, keep_active(rf, refill), fin);
+        if (active) step_run<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, rf.left <= 0, refill, fin);
     }
     n_ray   = wave_sum(n_ray);
     n_abort = wave_sum(n_abort);
@@ -911,14 +914,11 @@ __global__ void __launch_bounds__(256, DUAL ? 4 : 5)
             if (rp.left <= 0 && rs.left <= 0 && __ballot((tag & kTagPend) != 0u || fin != ST_CONT) == 0ull) break;
             continue;
         }
-        /* step until `keep` lanes are left: refill thresholds as in the two
+        /* step until so many lanes are idle: refill thresholds as tuned for the
          * separate launches; a wave with deferred lights returns as soon as
          * one ray ends, so that lane starts its next light */
-        const int keep = __ballot((tag & kTagPend) != 0u) ? 64
-                         : rp.left > 0                    ? 65 - (int) refill_p
-                         : rs.left > 0                    ? 65 - (int) refill_s
-                                                          : 1;
-        if (active) step_run<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, keep, fin);
+        const unsigned rule = __ballot((tag & kTagPend) != 0u) ? 1u : rp.left > 0 ? refill_p : rs.left > 0 ? refill_s : 64u;
+        if (active) step_run<CMP, DUAL, kSemShader, GRID>(s, r, st, t, active, false, rule, fin);
     }
     if (COUNT) n_exp = wave_sum(n_exp);
     if (lane == 0) {
@@ -1112,11 +1112,13 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
 
     const int      bs     = c->block_threads(s.maxlevel, DUAL);
     const size_t   lds    = (GSTK ? 0 : qbt_stack_bytes(s.maxlevel, DUAL, bs)) + sizeof(uint32_t) * kMailWords * bs;
-    /* refill thresholds: the tuned one for both launches, else the measured
-     * defaults (camera rays are shorter, so their refills cost more of a ray) */
+    /* refill: at the tuned number of idle lanes for every launch, else the
+     * measured defaults (refill_rule; camera rays are shorter than shadow
+     * rays, so their refills cost more of a ray) */
     const bool     tuned     = c->tune_refill > 0 && c->tune_refill <= 64;
-    const unsigned refill    = (unsigned) (tuned ? c->tune_refill : 24);
-    const unsigned refill_sh = (unsigned) (tuned ? c->tune_refill : 16);
+    const unsigned refill_sh = tuned ? (unsigned) c->tune_refill : 16u;
+    const unsigned refill_f  = tuned ? (unsigned) c->tune_refill : 24u; /* k_frame's camera rays */
+    const unsigned refill    = tuned ? (unsigned) c->tune_refill : refill_rule(48u, 180u);
     auto           kp     = k_primary<CMP, DUAL, GRID, COUNT, GSTK>;
     auto           ks     = k_shadow<CMP, DUAL, GRID, COUNT, GSTK>;
     auto           kf     = k_frame<CMP, DUAL, GRID, COUNT, GSTK>;
@@ -1167,7 +1169,7 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
             c->prof_mark_begin(QBT_PROF_FRAME);
             kf<<<gf, bs, lds, st>>>(s, b, po, L, nitems, nspr, c->tune_strip, (int*) c->sprite.p,
                                     (uint32_t*) c->wb_slots.p, (uint8_t*) c->wb_lstat.p, npix,
-                                    (unsigned*) c->wb_disc.p, q, refill, refill_sh, gstk, (int*) c->wb_lexp.p, cnt);
+                                    (unsigned*) c->wb_disc.p, q, refill_f, refill_sh, gstk, (int*) c->wb_lexp.p, cnt);
             c->prof_mark_end();
             k_shade<DUAL, COUNT><<<nblk(npix), 256, 0, st>>>(s, b, po, (const uint8_t*) c->wb_lstat.p,
                                                              (const int*) c->wb_lexp.p, npix, mask, cnt);
@@ -1226,7 +1228,7 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
     static_assert(sizeof(bp) == sizeof(key.bufs), "graph key buffers");
     memcpy(key.bufs, bp, sizeof(bp));
     key.nitems = nitems, key.npix = npix, key.nviews = (uint32_t) b.n, key.nlights = (uint32_t) nl;
-    key.mask = mask, key.flags = flags, key.bs = bs, key.refill = (int) (refill | refill_sh << 8), key.gp = gp, key.gs = gs;
+    key.mask = mask, key.flags = flags, key.bs = bs, key.refill = (int) refill, key.gp = gp, key.gs = gs;
     key.stack = GSTK, key.reorder = reorder, key.strip = c->tune_strip, key.gf = gf, key.merged = merged;
     memcpy(key.lights, L.p, sizeof(key.lights));
     key.tmpl = (CMP ? 1u : 0u) | (DUAL ? 2u : 0u) | (GRID ? 4u : 0u);

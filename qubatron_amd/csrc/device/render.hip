@@ -11,8 +11,9 @@
  *              order, views in order; writes the hit record (entry point,
  *              model indices, leaf, flags) and, per work item, the batch
  *              pixel index when the pixel is shaded
- *   k_sel_*    list of the shaded pixels in item order: per-block counts, a
- *              scan of the counts, scatter (no same-address atomics)
+ *   k_sel_*    list of the shaded pixels in item order: per-block counts,
+ *              their sums (in the next launch, or by a scan when the blocks
+ *              are many), scatter (no same-address atomics)
  *   k_oct_*    per light, the list partitioned by the direction octant of
  *              the shadow ray, list order kept within an octant (tuning
  *              reorder = 1)
@@ -93,6 +94,7 @@ struct PrimOut {
     uint8_t*  flags; /* QBT_PX_LEAF | QBT_PX_SHADED | QBT_PX_DISCARD */
     uint32_t* cand;  /* per work item: batch pixel index if shaded, else ~0 */
     int*      exp;   /* per pixel expansions (counting renders) */
+    unsigned* disc;  /* shaded pixels: the lowest light whose ray discarded the fragment, ~0 none so far */
 };
 
 /* the calling lane's traversal stack: LDS, or global memory (GSTK) */
@@ -177,7 +179,8 @@ __global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, Prim
             f    = QBT_PX_LEAF;
             if (isp.w > 0.0f) {
                 f |= QBT_PX_SHADED;
-                cand = gp;
+                cand       = gp;
+                o.disc[gp] = ~0u;
             }
         }
         o.isp[gp]        = isp;
@@ -351,14 +354,26 @@ __global__ void __launch_bounds__(1024) k_sel_scan(uint32_t* __restrict__ bcnt, 
 }
 
 /* values of the kept indices, in index order, at out + row * ostride */
-template <class P>
+template <class P, bool PRE>
 __global__ void __launch_bounds__(256) k_sel_scatter(P p, const uint32_t* __restrict__ boff, uint32_t nb,
-                                                     uint32_t* __restrict__ out, size_t ostride)
+                                                     uint32_t* __restrict__ out, size_t ostride,
+                                                     unsigned* __restrict__ total, int tstride)
 {
     __shared__ uint32_t ws[4];
     const int           row  = blockIdx.y;
     const int           lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    uint32_t            base = boff[(size_t) row * nb + blockIdx.x];
+    uint32_t            base;
+    if (PRE) { /* boff holds counts: this block's offset is the sum of those before it */
+        base = 0;
+        for (uint32_t i = threadIdx.x; i < blockIdx.x; i += 256) base += boff[(size_t) row * nb + i];
+        base = wave_sum(base);
+        if (lane == 0) ws[w] = base;
+        __syncthreads();
+        base = ws[0] + ws[1] + ws[2] + ws[3];
+        __syncthreads();
+    } else {
+        base = boff[(size_t) row * nb + blockIdx.x];
+    }
     for (int k = 0; k < kSelItems / 256; k++) {
         uint32_t       v    = 0;
         const bool     keep = p(blockIdx.x * kSelItems + k * 256 + threadIdx.x, row, v);
@@ -372,16 +387,32 @@ __global__ void __launch_bounds__(256) k_sel_scatter(P p, const uint32_t* __rest
         base += tot;
         __syncthreads();
     }
+    if (PRE && blockIdx.x + 1 == nb && threadIdx.x == 0) total[(size_t) row * tstride] = base;
 }
+
+/* Up to this many blocks of a compaction every block sums the counts before
+ * its own; beyond it they are scanned by a launch of their own. Summing costs
+ * the square of the blocks: 8.3M items (4051 blocks) 27.8 us with it against
+ * 13.7 + 8.5 us and a launch, but nothing that shows at 2.1M (1013 blocks),
+ * where the scan took 4.6 us and a launch: frame of 10M points 1143 -> 1128
+ * and 494 -> 480 us, together with the clearing of the discard words by
+ * k_primary; with surrogate decisions, two lists, 579 -> 545 us. */
+constexpr uint32_t kSelPrefix = 2048;
+inline uint32_t    sel_blocks(uint32_t n) { return (n + kSelItems - 1) / kSelItems + 1; }
+inline bool        sel_scans(uint32_t n) { return sel_blocks(n) > kSelPrefix; }
 
 template <class P>
 void compact(hipStream_t st, P p, uint32_t n, int rows, uint32_t* bcnt, unsigned* total, int tstride, uint32_t* out,
              size_t ostride)
 {
-    const uint32_t nb = (n + kSelItems - 1) / kSelItems + 1;
+    const uint32_t nb = sel_blocks(n);
     k_sel_count<P><<<dim3(nb, rows), 256, 0, st>>>(p, bcnt, nb);
+    if (!sel_scans(n)) {
+        k_sel_scatter<P, true><<<dim3(nb, rows), 256, 0, st>>>(p, bcnt, nb, out, ostride, total, tstride);
+        return;
+    }
     k_sel_scan<<<rows, 1024, 0, st>>>(bcnt, nb, total, tstride);
-    k_sel_scatter<P><<<dim3(nb, rows), 256, 0, st>>>(p, bcnt, nb, out, ostride);
+    k_sel_scatter<P, false><<<dim3(nb, rows), 256, 0, st>>>(p, bcnt, nb, out, ostride, total, tstride);
 }
 
 /* direction octant of the shadow ray light -> isp */
@@ -1147,6 +1178,7 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
     po.flags = (uint8_t*) c->wb_flags.p;
     po.cand  = (uint32_t*) c->wb_cand.p;
     po.exp   = (int*) c->wb_exp.p;
+    po.disc  = (unsigned*) c->wb_disc.p;
     unsigned*           q     = (unsigned*) c->wb_q.p;
     unsigned long long* cnt   = (unsigned long long*) c->counters.p;
     uint32_t*           items = (uint32_t*) c->wb_items.p;
@@ -1160,10 +1192,10 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
     auto enqueue = [&]() -> int {
         int err;
         k_zero_u32<<<nblk(Q_N), 256, 0, st>>>(q, Q_N);
-        k_fill_u32n<<<nblk(npix), 256, 0, st>>>((unsigned*) c->wb_disc.p, npix, ~0u);
         if (COUNT && nl > 0) /* lights the surrogate decided add no shadow expansions */
             k_fill_u32n<<<nblk((size_t) npix * nl), 256, 0, st>>>((unsigned*) c->wb_lexp.p, (size_t) npix * nl, 0u);
         if (merged) {
+            k_fill_u32n<<<nblk(npix), 256, 0, st>>>(po.disc, npix, ~0u);
             const size_t nw = (size_t) nitems * 4 * nl;
             k_fill_u32n<<<nblk(nw), 256, 0, st>>>((unsigned*) c->wb_slots.p, nw, kSlotFree);
             c->prof_mark_begin(QBT_PROF_FRAME);
@@ -1214,7 +1246,9 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
     if (!use_graph) {
         if ((rc = enqueue())) return rc;
         HIPCHK(hipGetLastError());
-        c->last.launches += merged ? 5 + (COUNT ? 1 : 0) : 6 + (nl > 0 ? 1 : 0) + (reorder ? 4 : 0) + (surrogate ? 4 : 0);
+        c->last.launches += merged ? 5 + (COUNT ? 1 : 0) : 5 + (nl > 0 ? 1 : 0) + (reorder ? 4 : 0) + (surrogate ? 3 : 0) +
+                                                               (sel_scans(nitems) ? 1 : 0) +
+                                                               (surrogate && sel_scans(npix) ? 1 : 0);
         return QBT_OK;
     }
 

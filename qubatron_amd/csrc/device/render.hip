@@ -118,11 +118,13 @@ __device__ __forceinline__ uint32_t* wave_mail(uint32_t* lds, int L)
  * b.sprite), then nitems pixel items.
  *
  * Bound by the issue of the traversal step's vector instructions and, towards
- * the end, by the latency of a lone wave's step. Five waves per SIMD (87
- * VGPRs): at six the slow paths spill, and 2.07M short rays take 313 us
- * against 304 (long ones, 8.3M of a 2160p frame, 5.32 against 5.51 ms). */
+ * the end, by the latency of a lone wave's step. Six waves per SIMD
+ * with one tree (80 VGPRs, 20 bytes of scratch outside the step's common
+ * path) against five (87): 8.3M long rays of a 2160p frame 4.79 against 4.98
+ * ms, 2.07M short ones 281 against 278 us; with both trees six take 193
+ * against 183 us on short rays, so five. */
 template <bool CMP, bool DUAL, bool GRID, bool COUNT, bool GSTK>
-__global__ void __launch_bounds__(256, 5) k_primary(SceneDev s, BatchDev b, PrimOut o, uint32_t nitems, uint32_t nspr,
+__global__ void __launch_bounds__(256, DUAL ? 5 : 6) k_primary(SceneDev s, BatchDev b, PrimOut o, uint32_t nitems, uint32_t nspr,
                                                  int nl, int strip, int* __restrict__ sprite, unsigned* __restrict__ q,
                                                  unsigned refill, GridRule rule, uint32_t* gstack,
                                                  unsigned long long* __restrict__ counters)
@@ -517,12 +519,12 @@ __global__ void k_oct_scan(const unsigned* __restrict__ cnt, unsigned* __restric
  * (lexp: per light, counting renders), so the frame does not depend on the
  * order in which rays end (the sample collector applies the same rule).
  *
- * Five waves per SIMD (91 VGPRs); six spill, and with a longer step (95
- * VGPRs) took 560 against 536 us on the shadow rays of a 1080p frame of 10M
- * points, 1.87 against 1.82 ms on a batch of 12 views, 8.49 against 8.58 ms
- * on a 2160p frame of 30M. */
+ * Six waves per SIMD with one tree (they spill outside the step's common
+ * path) against five (91 VGPRs): 6.66 against 6.88 ms on the shadow rays of a
+ * 2160p frame of 30M points, 1.98 against 2.00 ms at 1080p with 90M, 457
+ * against 453 us with 10M. */
 template <bool CMP, bool DUAL, bool GRID, bool COUNT, bool GSTK>
-__global__ void __launch_bounds__(256, 5)
+__global__ void __launch_bounds__(256, DUAL ? 5 : 6)
     k_shadow(SceneDev s, LightsDev L, const uint32_t* __restrict__ lists,
                                                 size_t lstride, const unsigned* __restrict__ counts, int cstride,
                                                 const float4* __restrict__ isp, uint8_t* __restrict__ lstat,
@@ -672,7 +674,7 @@ __device__ __forceinline__ uint32_t slot_xchg(uint32_t* p, uint32_t v)
 
 /* lane state of k_frame, packed into three words so that the kernel needs
  * few more registers than the separate launches (96 and a spill outside the
- * step against 91-95, 5 waves per SIMD; 4 waves without it: 3.39 against
+ * step, 5 waves per SIMD; 4 waves without it: 3.39 against
  * 3.27 ms on a 1080p frame of 90M points): gp = the ray's batch pixel; k = the camera ray's work
  * item, or the shadow ray's slot; tag = kind bits, the sprite slot of a
  * sprite trace, and the lights still deferred to this lane (bits 8..15) */

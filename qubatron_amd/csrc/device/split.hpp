@@ -315,8 +315,8 @@ __device__ __forceinline__ void step_run(const SceneDev& s, const Ray& r, const 
 }
 
 /* Blocks of a persistent traversal launch over at most `items` rays: all
- * that are resident (5 waves per SIMD for the traversal kernels: VGPRs and LDS
- * stacks), at most one lane per ray, but not fewer than
+ * that are resident (5 or 6 waves per SIMD for the traversal kernels: VGPRs and
+ * LDS stacks), at most one lane per ray, but not fewer than
  * kSpreadWavesPerSimd waves per SIMD: those then take fewer rays each
  * (Refill::share), down to one. A wave alone on its SIMD steps at its own
  * latency, so a second one is nearly free, and the lanes without a ray take

@@ -605,13 +605,14 @@ __device__ __forceinline__ uint32_t expand_any(const SceneDev& s, const Ray& r, 
  * octet by coordinates, and its tie-flipped octet where that equals the one
  * before, come to the same), and the sort needs the keys alone. false where
  * any of this does not hold: the caller takes expand_any. The traversal of
- * large frames is bound by the issue of vector instructions (180 to 205 node
+ * large frames is bound by the issue of vector instructions (190 to 225 node
  * expansions per ns), so the step is written for their number: 118 to here
  * against 173 of expand_any and the checks of its quotients, one rare branch
  * instead of four. k_primary + k_shadow of a 2160p frame of 30M points took
  * 15.38 ms with expand_any alone, 15.07 with a first form of this (the keys
- * from the hits' coordinates, 135 instructions; 62 in plane_entry), 12.83 now
- * (44 in plane_entry); 200k free rays 238, 209 and 190 us. */
+ * from the hits' coordinates, 135 instructions; 62 in plane_entry), 12.83 with
+ * 118 and 44, 11.88 with 35 in plane_entry (the root's entry and ancestors'
+ * planes off its common path); 200k free rays 238, 209, 190 and 183 us. */
 __device__ __forceinline__ bool expand_general_position(const SceneDev& s, const Ray& r, const TraceState& t,
                                                         uint32_t mask, uint32_t& word, int& n)
 {
@@ -663,37 +664,41 @@ __device__ __forceinline__ bool expand_general_position(const SceneDev& s, const
     return !bad;
 }
 
-/* Entry point of the child behind `plane` (1 x, 2 y, 3 or 4 z) of the node at
- * level j whose cell coordinates are (ix, iy, iz) >> sh, or, plane 0, the
- * root entry: midplane_cell's and root_entry's, the quotient unchecked where
- * the ray allows. On an exact grid the mid-plane's coordinate is one FMA:
- * base +- (2 i + 1) w / 2 is a number that fp32 holds; the root's faces are
- * base and base +- 2 w / 2 (j = 0), rounded as root_entry's sum. */
-template <int SEM, bool GRID>
-__device__ __forceinline__ float4 plane_entry(const SceneDev& s, const Ray& r, const TraceState& t, int plane, int j,
-                                              int sh)
+/* Entry point of an entry whose plane is `plane` (1 x, 2 y, 3 or 4 z) of the
+ * node at level lv of the path, with cell coordinates (sx, sy, sz):
+ * midplane_cell's, the quotient unchecked where the ray allows. On an exact
+ * grid the mid-plane's coordinate is one FMA: base +- (2 i + 1) w / 2 is a
+ * number that fp32 holds. Plane 0, the node's own entry point (a backtracking
+ * lane needs it in rare orders of a node's candidates only): the mid-plane hit
+ * of the nearest node on the path entered through one (plane_of reads that of
+ * a level), else the root entry. */
+template <int SEM, bool GRID, class PlaneOf>
+__device__ __forceinline__ float4 plane_entry(const SceneDev& s, const Ray& r, const TraceState& t, int plane, int lv,
+                                              int sx, int sy, int sz, PlaneOf&& plane_of)
 {
-    if (!GRID || (t.pend & kSlowRay) != 0u)
+    if (!GRID || plane == 0 || (t.pend & kSlowRay) != 0u) {
+        int j = lv;
+        while (plane == 0 && j > 0) {
+            j--;
+            plane = plane_of(j);
+        }
         return plane == 0 ? root_entry<SEM>(s, r, root_face(t))
-                          : midplane_cell<SEM, GRID>(s, r, plane == 1 ? 2 : (plane == 2 ? 3 : 1), j, t.ix, t.iy, t.iz, sh);
-    const bool root = plane == 0;
-    const int  f = root_face(t), at = root ? f & 3 : plane;
-    const bool px = at == 1, py = at == 2, in = at == 0;
-    const int  i = sel(px, t.ix, sel(py, t.iy, t.iz)) >> sh;
-    const int  m = root ? (f >> 1) & 2 : 2 * i + 1;
-    const float h = ldexpf(s.bw, -1 - j);
+                          : midplane_cell<SEM, GRID>(s, r, plane == 1 ? 2 : (plane == 2 ? 3 : 1), j, sx, sy, sz, lv - j);
+    }
+    const bool  px = plane == 1, py = plane == 2;
+    const int   m  = 2 * sel(px, sx, sel(py, sy, sz)) + 1;
+    const float h = ldexpf(s.bw, -1 - lv);
     const float bx = s.bx, by = s.by, bz = s.bz;
     const float c = __builtin_fmaf((float) m, px ? h : -h, px ? bx : (py ? by : bz));
     /* values, not the ray's members: a select between members is a load from
      * a selected address, and the ray then lives in memory */
     const float ox = r.px, oy = r.py, oz = r.pz, dx = r.dx, dy = r.dy, dz = r.dz, jx = r.ix, jy = r.iy, jz = r.iz;
-    float       q = quot(c, px ? ox : (py ? oy : oz), px ? dx : (py ? dy : dz), px ? jx : (py ? jy : jz));
-    q             = in ? 0.0f : q;
+    const float q = quot(c, px ? ox : (py ? oy : oz), px ? dx : (py ? dy : dz), px ? jx : (py ? jy : jz));
     const float X = r.px + r.dx * q, Y = r.py + r.dy * q, Z = r.pz + r.dz * q;
     float4      o;
     o.x = px ? c : X;
     o.y = py ? c : Y;
-    o.z = (px || py || in) ? Z : c;
+    o.z = (px || py) ? Z : c;
     o.w = q;
     return o;
 }
@@ -720,7 +725,7 @@ __device__ __forceinline__ int trace_step_c1(const SceneDev& s, const Ray& r, co
      * stack words every lane reads and rewrites, and the new words, the
      * pending mask and the child block are selects. */
     const bool     desc  = n > 0;
-    const uint32_t below = t.pend & ((1u << level) - 1u);
+    const uint32_t below = t.pend & ~kRayBits; /* levels at and below this one have none */
     if (!desc && below == 0u) return ST_MISS;
     /* the deepest level with a pending entry, from the per-lane mask (levels
      * between it and this one have none: no loop over them) */
@@ -736,24 +741,18 @@ __device__ __forceinline__ int trace_step_c1(const SceneDev& s, const Ray& r, co
     /* bit lv: whether the level still has a pending entry */
     t.pend = (t.pend & ~(1u << lv)) | (nw >= 1u << 30 ? 1u << lv : 0u);
     const uint32_t a = nw & 0x3FFFFFFFu;
-    /* Its entry point. Plane 0 (the node's own entry point): a descending
-     * lane keeps its entry; a backtracking one takes the mid-plane hit of the
-     * nearest node on the path entered through a mid-plane, else the root
-     * entry. Else that mid-plane of the level-j node, recomputed from the
-     * plane (same operations as the candidate, so the same bits). */
-    int j = lv, plane = (int) ((w >> 3) & 7u);
-    if (!desc && plane == 0) {
-        while (plane == 0 && j > 0) {
-            j--;
-            plane = (int) ((st.pw[st.at(j)] >> 3) & 7u);
-        }
-    }
-    if (!desc || plane != 0) t.entry = plane_entry<SEM, GRID>(s, r, t, plane, j, level - j);
-    const int sh = level - lv, o = (int) (w & 7u);
+    /* Its entry point: a descending lane with plane 0 keeps its own; else that
+     * of the plane, recomputed (same operations as the candidate, so the same
+     * bits). */
+    const int plane = (int) ((w >> 3) & 7u), sh = level - lv, o = (int) (w & 7u);
+    const int sx = t.ix >> sh, sy = t.iy >> sh, sz = t.iz >> sh;
+    if (!desc || plane != 0)
+        t.entry = plane_entry<SEM, GRID>(s, r, t, plane, lv, sx, sy, sz,
+                                         [&](int l) { return (int) ((st.pw[st.at(l)] >> 3) & 7u); });
     t.ns    = (int) (a + (uint32_t) __popc(__builtin_amdgcn_ubfe(w, 24u, (uint32_t) o))); /* first + rank */
-    t.ix    = ((t.ix >> sh) << 1) | (o & 1);
-    t.iy    = ((t.iy >> sh) << 1) | ((o >> 1) & 1);
-    t.iz    = ((t.iz >> sh) << 1) | (o >> 2);
+    t.ix    = (sx << 1) | (o & 1);
+    t.iy    = (sy << 1) | ((o >> 1) & 1);
+    t.iz    = (sz << 1) | (o >> 2);
     t.level = lv + 1;
     return t.level == s.maxlevel ? ST_HIT : ST_CONT;
 }
@@ -774,17 +773,13 @@ __device__ __forceinline__ int trace_pop_c1(const SceneDev& s, const Ray& r, con
     st.pw[at] = w;
     st.ns[at] = (int) (an - (1u << 30));
     t.pend ^= an - (1u << 30) >= 1u << 30 ? 0u : 1u << lv;
-    int j = lv, plane = (int) ((w >> 3) & 7u);
-    while (plane == 0 && j > 0) {
-        j--;
-        plane = (int) ((st.pw[st.at(j)] >> 3) & 7u);
-    }
-    t.entry      = plane_entry<SEM, GRID>(s, r, t, plane, j, level - j);
-    const int sh = level - lv, o = (int) (w & 7u);
+    const int sh = level - lv, o = (int) (w & 7u), sx = t.ix >> sh, sy = t.iy >> sh, sz = t.iz >> sh;
+    t.entry = plane_entry<SEM, GRID>(s, r, t, (int) ((w >> 3) & 7u), lv, sx, sy, sz,
+                                     [&](int l) { return (int) ((st.pw[st.at(l)] >> 3) & 7u); });
     t.ns    = (int) ((an & 0x3FFFFFFFu) + (uint32_t) __popc(__builtin_amdgcn_ubfe(w, 24u, (uint32_t) o)));
-    t.ix    = ((t.ix >> sh) << 1) | (o & 1);
-    t.iy    = ((t.iy >> sh) << 1) | ((o >> 1) & 1);
-    t.iz    = ((t.iz >> sh) << 1) | (o >> 2);
+    t.ix    = (sx << 1) | (o & 1);
+    t.iy    = (sy << 1) | ((o >> 1) & 1);
+    t.iz    = (sz << 1) | (o >> 2);
     t.level = lv + 1;
     return t.level == s.maxlevel ? ST_HIT : ST_CONT;
 }
@@ -821,25 +816,21 @@ __device__ __forceinline__ int enter_c2(const SceneDev& s, const Ray& r, const S
                                         int lv, uint32_t e, uint32_t pw, uint32_t an, uint32_t ad)
 {
     const int at = st.at(lv), level = t.level;
-    int       j = lv, plane = (int) plane_code(e);
+    const int plane = (int) plane_code(e), sh = level - lv, o = (int) (e & 7u);
+    const int sx = t.ix >> sh, sy = t.iy >> sh, sz = t.iz >> sh;
     st.pw[at] = pw;
     st.ns[at] = (int) (an | (uint32_t) plane << 30);
     st.nd[at] = (int) ad;
-    if (!keep) {
-        while (plane == 0 && j > 0) {
-            j--;
-            plane = (int) ((uint32_t) st.ns[st.at(j)] >> 30);
-        }
-    }
-    if (!keep || plane != 0) t.entry = plane_entry<SEM, GRID>(s, r, t, plane, j, level - j);
-    const int      sh = level - lv, o = (int) (e & 7u);
+    if (!keep || plane != 0)
+        t.entry = plane_entry<SEM, GRID>(s, r, t, plane, lv, sx, sy, sz,
+                                         [&](int l) { return (int) ((uint32_t) st.ns[st.at(l)] >> 30); });
     const uint32_t cs = an + (uint32_t) __popc(__builtin_amdgcn_ubfe(pw, 24u, (uint32_t) o));
     const uint32_t cd = (ad & 0xFFFFFFu) + (uint32_t) __popc(__builtin_amdgcn_ubfe(ad, 24u, (uint32_t) o));
     t.ns    = (e & 64u) ? (int) cs : 0;
     t.nd    = (e & 128u) ? (int) cd : 0;
-    t.ix    = ((t.ix >> sh) << 1) | (o & 1);
-    t.iy    = ((t.iy >> sh) << 1) | ((o >> 1) & 1);
-    t.iz    = ((t.iz >> sh) << 1) | (o >> 2);
+    t.ix    = (sx << 1) | (o & 1);
+    t.iy    = (sy << 1) | ((o >> 1) & 1);
+    t.iz    = (sz << 1) | (o >> 2);
     t.level = lv + 1;
     return t.level == s.maxlevel ? ST_HIT : ST_CONT;
 }
@@ -857,7 +848,7 @@ __device__ __forceinline__ int trace_step_c2(const SceneDev& s, const Ray& r, co
     if (!GRID || !expand_general_position(s, r, t, ms | md, word, n)) word = expand_any<SEM, GRID>(s, r, t, ms | md, n);
 
     const bool     desc  = n > 0;
-    const uint32_t below = t.pend & ((1u << level) - 1u);
+    const uint32_t below = t.pend & ~kRayBits; /* levels at and below this one have none */
     if (!desc && below == 0u) return ST_MISS;
     const int      lv  = desc ? level : top_bit(below);
     const int      at  = st.at(lv);

@@ -605,7 +605,7 @@ __device__ __forceinline__ uint32_t expand_any(const SceneDev& s, const Ray& r, 
  * octet by coordinates, and its tie-flipped octet where that equals the one
  * before, come to the same), and the sort needs the keys alone. false where
  * any of this does not hold: the caller takes expand_any. The traversal of
- * large frames is bound by the issue of vector instructions (190 to 225 node
+ * large frames is bound by the issue of vector instructions (195 to 225 node
  * expansions per ns), so the step is written for their number: 118 to here
  * against 173 of expand_any and the checks of its quotients, one rare branch
  * instead of four. k_primary + k_shadow of a 2160p frame of 30M points took

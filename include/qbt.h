@@ -322,7 +322,10 @@ int qbt_particle_update(qbt_ctx* ctx, const float* pos, const float* spd, size_t
  * build (a per-frame rebuild then allocates nothing); a static build releases
  * its scratch when it ends. Kept scratch counts against max_device_bytes; it
  * is released when another allocation of the context would exceed that cap
- * or find the device full, and by qbt_destroy. */
+ * or find the device full, and by qbt_destroy. A build refused for its points
+ * or its scratch (QBT_ERANGE, QBT_ENOTSUP, QBT_ENOMEM) leaves the tree as it
+ * was; one that fails once the node array is being replaced (QBT_ENOMEM,
+ * QBT_EDEVICE) leaves no tree, until one is uploaded or built. */
 int qbt_build_octree(qbt_ctx* ctx, int tree, const float basecube[4], int levels, size_t npoints,
                      size_t* nodes_out);
 

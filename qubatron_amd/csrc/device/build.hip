@@ -468,19 +468,25 @@ static int build_t(qbt_ctx* c, int t, float edge, int levels, size_t n, size_t* 
     }
     /* 2. the arrays: the node array and, unless its 30-bit first-child
      * indices overflow, the compact layout (its arrays hold the records
-     * while the tree is built; scratch does otherwise) */
+     * while the tree is built; scratch does otherwise). The arrays are
+     * replaced or overwritten from here on, and nothing clears them first: a
+     * build that fails below leaves no tree, and what a later upload does not
+     * write is checked and laid out as new */
+    const bool cmp = total < (1u << 30);
+    tr.n           = 0;
+    tr.validated   = false;
+    tr.full_check  = true;
+    tr.cmp_stale   = true;
+    tr.patch.clear();
+    cm.ok = false, cm.n = 0, cm.ref_n = 0;
     if (total > tr.cap_nodes) {
         const size_t cap = total + total / 4 + 1024;
         c->dev_free(tr.child);
         c->dev_free(tr.model);
         tr.cap_nodes = 0;
-        tr.n         = 0;
         if ((rc = c->dev_alloc(tr.child, cap * 32)) || (rc = c->dev_alloc(tr.model, cap * 4))) return rc;
         tr.cap_nodes = cap;
     }
-    const bool cmp = total < (1u << 30);
-    cm.ok = false, cm.n = 0, cm.ref_n = 0;
-    tr.n  = total; /* compact_reserve sizes the reference map by it */
     uint2* rec;
     int *  model_c, *ref, *r2c;
     if (cmp) {
@@ -519,12 +525,12 @@ static int build_t(qbt_ctx* c, int t, float edge, int levels, size_t n, size_t* 
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s));
     /* every child index above is a node index below total: nothing to check */
+    tr.n          = total;
     tr.validated  = true;
     tr.full_check = false;
     tr.dirty_lo = tr.dirty_hi = 0;
     tr.vdirty.clear();
     tr.vdirty_over = false;
-    tr.patch.clear();
     tr.cmp_stale = !cmp;
     if (cmp) cm.ok = true, cm.n = total, cm.ref_n = total;
     if (nodes_out) *nodes_out = total;

@@ -399,12 +399,14 @@ int qbt_ctx::compact_reserve(int t, size_t nrec, size_t nref)
     int          rc;
     if (nrec > cm.cap) { /* room for the records in-place patches append */
         const size_t cap = nrec + nrec / 8 + 65536;
+        cm.cap           = 0; /* a failed allocation may leave one of the three without memory */
         if ((rc = dev_alloc(cm.rec, cap * 8)) || (rc = dev_alloc(cm.model, cap * 4)) || (rc = dev_alloc(cm.ref, cap * 4)))
             return rc;
         cm.cap = cap;
     }
     if (nref > cm.r2c_cap) {
         const size_t cap = nref > tree[t].cap_nodes ? nref : tree[t].cap_nodes;
+        cm.r2c_cap       = 0;
         if ((rc = dev_alloc(cm.r2c, cap * 4))) return rc;
         cm.r2c_cap = cap;
     }

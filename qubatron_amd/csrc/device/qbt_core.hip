@@ -1026,7 +1026,7 @@ int qbt_ctx::scene_for(const float basecube[4], int maxlevel, SceneDev& s, bool&
                 tb.cmp_stale = false;
             }
         }
-        cmp = tree[0].cmp.ok && (!dual || (tree[1].cmp.ok && tree[1].cmp.n < kDualRecords));
+        cmp = tree[0].cmp.ok && (!dual || tree[1].cmp.ok);
     }
     memset(&s, 0, sizeof(s));
     for (int t = 0; t < 2; t++) {
@@ -1043,6 +1043,7 @@ int qbt_ctx::scene_for(const float basecube[4], int maxlevel, SceneDev& s, bool&
     s.bx = basecube[0], s.by = basecube[1], s.bz = basecube[2], s.bw = basecube[3];
     s.maxlevel = maxlevel;
     s.iter_cap = iter_cap;
+    s.dyn_wide = cmp && dual && tree[1].cmp.n >= kDualRecords;
     return QBT_OK;
 }
 

@@ -76,6 +76,7 @@ struct SceneDev {
     float bx, by, bz, bw; /* basecube */
     int maxlevel;
     int iter_cap;
+    int dyn_wide; /* both trees on compact layouts, the dynamic one of kDualRecords records or more (trace_step_c2) */
 };
 
 struct Ray {
@@ -381,8 +382,8 @@ struct TraceState {
 
 enum : int { ST_CONT = 2 };
 
-/* records a dynamic compact layout may have when both trees are walked
- * (trace_step_c2's stack words) */
+/* from this many records of the dynamic compact layout on, a stack word does
+ * not hold a first child beside the block's slots (trace_step_c2) */
 constexpr uint32_t kDualRecords = 1u << 24;
 
 constexpr uint32_t kSlowRay   = 0x80000000u; /* in pend: the ray's quotients need plane_k's check */
@@ -794,13 +795,16 @@ __device__ __forceinline__ int trace_pop_c1(const SceneDev& s, const Ray& r, con
  *            node's slots
  *   ns word  the static node's first child (30 bits) | the plane of the entry
  *            being visited << 30 (1 x, 2 y, 3 z, 0 the node's entry point)
- *   nd word  the dynamic node's first child (24 bits) | its slots << 24
- * so the dynamic layout has fewer than kDualRecords records; beyond that both
- * trees are walked on the direct layout. A node index is 0 where the path has
- * left its tree. Against the direct layout's step on compact records (separate
+ *   nd word  the dynamic node's first child (24 bits) | its slots << 24; with
+ *            kDualRecords records or more (SceneDev::dyn_wide) the node's
+ *            index, and its record is read again on a backtrack
+ * A node index is 0 where the path has left its tree. Against the direct layout's step on compact records (separate
  * descend and backtrack paths, records read again on a backtrack), 720p over
  * 5M static and 150k dynamic points: k_primary 633 -> 548 us, 719 -> 603 and
- * 202 -> 200 (three poses), k_shadow 292 -> 247, 403 -> 342, 96 -> 88.
+ * 202 -> 200 (three poses), k_shadow 292 -> 247, 403 -> 342, 96 -> 88. Frames
+ * of 5M static points and 28.9M dynamic records (the wide words): 0.64, 0.79
+ * and 1.18 ms, against 0.89, 1.09 and 1.80 with both trees on the direct
+ * layout; the test of dyn_wide costs narrow frames nothing (within 0.3%).
  */
 /* the plane of an entry's bits 3-5 (one-hot) as a number: 1 x, 2 y, 3 z */
 __device__ __forceinline__ uint32_t plane_code(uint32_t e)
@@ -810,22 +814,29 @@ __device__ __forceinline__ uint32_t plane_code(uint32_t e)
 }
 
 /* the second half of a step: entry e (8 bits) of level lv becomes the current
- * one; an, pw and ad are that level's new words (an without the plane) */
+ * one; an, pw and ad are that level's new words (an without the plane; ad of
+ * a descending lane, keep, as the narrow form has it), rd the dynamic node's
+ * record where the lane descends */
 template <int SEM, bool GRID>
 __device__ __forceinline__ int enter_c2(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t, bool keep,
-                                        int lv, uint32_t e, uint32_t pw, uint32_t an, uint32_t ad)
+                                        int lv, uint32_t e, uint32_t pw, uint32_t an, uint32_t ad, uint2 rd)
 {
     const int at = st.at(lv), level = t.level;
     const int plane = (int) plane_code(e), sh = level - lv, o = (int) (e & 7u);
     const int sx = t.ix >> sh, sy = t.iy >> sh, sz = t.iz >> sh;
     st.pw[at] = pw;
     st.ns[at] = (int) (an | (uint32_t) plane << 30);
-    st.nd[at] = (int) ad;
     if (!keep || plane != 0)
         t.entry = plane_entry<SEM, GRID>(s, r, t, plane, lv, sx, sy, sz,
                                          [&](int l) { return (int) ((uint32_t) st.ns[st.at(l)] >> 30); });
     const uint32_t cs = an + (uint32_t) __popc(__builtin_amdgcn_ubfe(pw, 24u, (uint32_t) o));
-    const uint32_t cd = (ad & 0xFFFFFFu) + (uint32_t) __popc(__builtin_amdgcn_ubfe(ad, 24u, (uint32_t) o));
+    uint32_t       cd = (ad & 0xFFFFFFu) + (uint32_t) __popc(__builtin_amdgcn_ubfe(ad, 24u, (uint32_t) o));
+    if (s.dyn_wide) { /* uniform */
+        if (keep) ad = (uint32_t) t.nd;
+        else rd = s.dyn.rec[ad];
+        cd = rd.x + (uint32_t) __popc(__builtin_amdgcn_ubfe(rd.y, 8u, (uint32_t) o));
+    }
+    st.nd[at] = (int) ad;
     t.ns    = (e & 64u) ? (int) cs : 0;
     t.nd    = (e & 128u) ? (int) cd : 0;
     t.ix    = (sx << 1) | (o & 1);
@@ -867,7 +878,7 @@ __device__ __forceinline__ int trace_step_c2(const SceneDev& s, const Ray& r, co
     /* bit lv: whether the level still has a pending entry */
     t.pend = (t.pend & ~(1u << lv)) | ((w & 0xFFFFFFu) != 0u ? 1u << lv : 0u);
     return enter_c2<SEM, GRID>(s, r, st, t, desc, lv, e, w, desc ? rs.x : an & 0x3FFFFFFFu,
-                               desc ? (rd.x & 0xFFFFFFu) | (rd.y >> 8) << 24 : ad);
+                               desc ? (rd.x & 0xFFFFFFu) | (rd.y >> 8) << 24 : ad, rd);
 }
 
 /* the backtrack half of trace_step_c2 (as trace_pop_c1) */
@@ -879,7 +890,7 @@ __device__ __forceinline__ int trace_pop_c2(const SceneDev& s, const Ray& r, con
     const uint32_t pwv = st.pw[at], an = (uint32_t) st.ns[at], ad = (uint32_t) st.nd[at];
     const uint32_t w   = ((pwv & 0xFFFFFFu) >> 8) | (pwv & 0xFF000000u);
     t.pend ^= ((w & 0xFFFFFFu) != 0u ? 0u : 1u) << lv;
-    return enter_c2<SEM, GRID>(s, r, st, t, false, lv, pwv & 0xFFu, w, an & 0x3FFFFFFFu, ad);
+    return enter_c2<SEM, GRID>(s, r, st, t, false, lv, pwv & 0xFFu, w, an & 0x3FFFFFFFu, ad, make_uint2(0u, 0u));
 }
 
 /* backtrack (octree_fsh.c:368-375) and pop the next pending entry of the

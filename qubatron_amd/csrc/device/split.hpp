@@ -35,6 +35,13 @@
  *
  * Every step of the loop takes a segment further or ends it, no lane waits
  * for another inside a burst, and the loop ends when no ray is left.
+ *
+ * The iteration cap is that of the serial trace (near_cap), which takes no
+ * more steps than a ray's segments together, at most 64 kBurst a round. So
+ * rays are shared for half the cap's worth of rounds, if none of the wave has
+ * used the other half up; a ray that still has no result then (it would take
+ * a path of hundreds of thousands of nodes, or an array that is no tree)
+ * starts again, unshared, and its steps are counted.
  */
 #pragma once
 
@@ -89,14 +96,17 @@ __device__ __forceinline__ void drain(const SceneDev& s, Ray& r, const Stack& st
     int       seg  = active ? (int) ST_CONT : kSegFree;
     int       own  = lane;
     uint32_t  a = 0, b = kKeyEnd;
+    int       rounds = s.iter_cap / (2 * 64 * kBurst); /* left with sharing; none: rays are whole */
+    if (__ballot(active && t.it > s.iter_cap / 2) != 0ull) rounds = 0;
     while (__ballot(live) != 0ull) {
+        const int burst = __ballot(seg == ST_CONT && near_cap<CMP>(s, t, kBurst)) != 0ull ? 1 : kBurst;
         if (seg == ST_CONT) {
 #pragma nounroll
-            for (int k = 0; k < kBurst; k++) {
+            for (int k = 0; k < burst; k++) {
                 seg = trace_step<CMP, DUAL, SEM, GRID>(s, r, st, t);
                 if (seg != ST_CONT) break;
             }
-            if (count_steps<CMP, DUAL>(s, t, kBurst) && seg == ST_CONT) seg = ST_ABORT;
+            if (count_steps<CMP, DUAL>(s, t, burst)) seg = ST_ABORT;
         }
         /* the lowest hit of every ray (an aborted segment ends its ray like a
          * hit), then its lowest unfinished key */
@@ -134,10 +144,19 @@ __device__ __forceinline__ void drain(const SceneDev& s, Ray& r, const Stack& st
                 if (live) seg = ST_CONT, a = 0, b = kKeyEnd;
             }
         }
+        if (rounds > 0 && --rounds == 0) { /* the unfinished rays again, whole */
+            seg = kSegFree;
+            if (live) {
+                t.entry = root_entry<SEM>(s, r, root_face(t));
+                t.level = t.ix = t.iy = t.iz = t.ns = t.nd = t.it = 0;
+                t.pend &= kRayBits;
+                seg = ST_CONT, a = 0, b = kKeyEnd;
+            }
+        }
         /* share */
         if (seg == kSegFree) own = lane;
         const uint32_t below = t.pend & ((1u << t.level) - 1u);
-        const bool     gives = seg == ST_CONT && below != 0u && b - a >= 2u;
+        const bool     gives = rounds > 0 && seg == ST_CONT && below != 0u && b - a >= 2u;
         const bool     idle  = seg == kSegFree && !live;
         const uint64_t gmask = __ballot(gives), imask = __ballot(idle);
         const int      pairs = min((int) __popcll(gmask), (int) __popcll(imask));
@@ -288,13 +307,14 @@ __host__ __device__ __forceinline__ constexpr unsigned refill_rule(unsigned lane
  * all such lanes together at the next refill point (a lane that ends would
  * otherwise run the output code with one or two lanes of its wave, in most
  * steps). */
-constexpr int kRunSteps = 4096; /* most steps between two looks at the iteration cap */
+constexpr int kRunSteps = 4096; /* most steps of a run (near_cap) */
 
 template <bool CMP, bool DUAL, int SEM, bool GRID, bool WASTE = false>
 __device__ __forceinline__ void step_run(const SceneDev& s, const Ray& r, const Stack& st, TraceState& t, bool& active,
                                          bool dry, unsigned rule, int& fin)
 {
     const int keep = dry ? 1 : 65 - (int) (rule & 255u), most = dry || rule < 256u ? INT_MAX : (int) (rule >> 8);
+    const int run = __ballot(near_cap<CMP>(s, t, kRunSteps)) != 0ull ? 1 : kRunSteps;
     int       steps = 0, waste = 0; /* of the wave in this call: uniform */
     for (;;) {
         const int stt = trace_step<CMP, DUAL, SEM, GRID>(s, r, st, t);
@@ -306,9 +326,9 @@ __device__ __forceinline__ void step_run(const SceneDev& s, const Ray& r, const 
         }
         const int on = (int) __popcll(__ballot(1));
         if (WASTE) waste += 64 - on;
-        if (on < keep || (WASTE && waste >= most) || steps == kRunSteps) break;
+        if (on < keep || (WASTE && waste >= most) || steps == run) break;
     }
-    if (count_steps<CMP, DUAL>(s, t, steps) && active) {
+    if (count_steps<CMP, DUAL>(s, t, steps)) {
         fin    = ST_ABORT;
         active = false;
     }

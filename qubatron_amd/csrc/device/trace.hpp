@@ -1043,8 +1043,19 @@ __device__ __forceinline__ int trace_pop(const SceneDev& s, const Ray& r, const 
     else return trace_pop_direct<DUAL, SEM, GRID>(s, r, st, t);
 }
 
-/* Counts the steps just taken (steps that do not count themselves) and
- * returns whether the ray is over the iteration cap. */
+/* The iteration cap: a ray whose trace takes more than iter_cap steps is
+ * aborted, whatever its last step came to. The direct layout's step counts
+ * itself; that of the compact ones is counted by its callers, a run of steps
+ * at a time. Only lanes far enough from the cap for a whole run take one
+ * (near_cap: all lanes of the wave then go one step at a time), so the count
+ * of a lane that may be over is its own. */
+template <bool CMP>
+__device__ __forceinline__ bool near_cap(const SceneDev& s, const TraceState& t, int run)
+{
+    return CMP && t.it > s.iter_cap - run;
+}
+
+/* counts the `steps` of the run just taken; whether the ray is over the cap */
 template <bool CMP, bool DUAL>
 __device__ __forceinline__ bool count_steps(const SceneDev& s, TraceState& t, int steps)
 {
@@ -1069,7 +1080,7 @@ __device__ int trace(const SceneDev& s, const Ray& r, const Stack& st, Hit& out)
     int        stt = trace_begin<SEM>(s, rr, t);
     while (stt == ST_CONT) {
         stt = trace_step<CMP, DUAL, SEM, GRID>(s, rr, st, t);
-        if (count_steps<CMP, DUAL>(s, t, 1) && stt == ST_CONT) stt = ST_ABORT;
+        if (count_steps<CMP, DUAL>(s, t, 1)) stt = ST_ABORT;
     }
     out.exps = t.exps;
     if (stt == ST_HIT) {

@@ -473,6 +473,7 @@ static int build_t(qbt_ctx* c, int t, float edge, int levels, size_t n, size_t* 
      * build that fails below leaves no tree, and what a later upload does not
      * write is checked and laid out as new */
     const bool cmp = total < (1u << 30);
+    if ((rc = c->flush_pending(t, true))) return rc; /* held uploads go with the old array */
     tr.n           = 0;
     tr.validated   = false;
     tr.full_check  = true;
@@ -546,8 +547,6 @@ extern "C" int qbt_build_octree(qbt_ctx* c, int tree, const float basecube[4], i
     const int t = tree == QBT_BUFFER_STATIC_OCTREE ? 0 : 1;
     if (npoints > c->pts[t].n || npoints >= (size_t) UINT32_MAX) return QBT_EINVAL;
     HIPCHK(hipSetDevice(c->device));
-    int rc;
-    if ((rc = c->flush_pending(t, true))) return rc; /* the build replaces the array */
     return 3 * levels <= 32 ? build_t<uint32_t>(c, t, basecube[3], levels, npoints, nodes_out)
                             : build_t<uint64_t>(c, t, basecube[3], levels, npoints, nodes_out);
 }

@@ -76,6 +76,23 @@ def test_static_build_out_of_memory(before):
         assert all(k == "exp" or x == 0 for k, x in mm.items()), mm
 
 
+def test_refused_build_keeps_held_uploads(gpu_ctx):
+    """A build refused for its points leaves the tree as it was, with the single-node uploads that the context still
+    holds back."""
+    bc = np.array([0.0, 1800.0, 1800.0, 1800.0], np.float32)
+    nodes = q.octree_from_points(np.random.default_rng(2).uniform(1, 1799, (500, 3)).astype(np.float32), bc, 6).nodes()
+    gpu_ctx.upload_octree(nodes)
+    edited = nodes.copy()
+    i, o = np.argwhere(nodes[:, :8] > 0)[40]
+    edited[i, o] = 0
+    gpu_ctx.upload_octree(edited, start_node=int(i), end_node=int(i) + 1)
+    gpu_ctx.upload_points(np.array([[-1000.0, 1000.0, 1000.0]], np.float32))  # an octet of -1
+    with pytest.raises(q.QbtError) as e:
+        gpu_ctx.build_octree(bc, 4, 1)
+    assert e.value.code == q._ffi.QBT_ERANGE
+    assert np.array_equal(gpu_ctx.download_octree(nodes.shape[0]), edited)
+
+
 def test_upload_after_a_failed_build():
     """An array uploaded into the memory that the failed build allocated."""
     sc, pnt, nrm, col, nodes = H.scene(1, npoints=100000)

@@ -233,11 +233,11 @@ int qbt_profile_end(qbt_ctx* ctx, qbt_profile* out);
  * and shadow rays back to back), 1 = wavefront stages with persistent,
  * lane-refilling traversal kernels over a batch of views. block_threads:
  * 64..256 (0 = default 256; halved while the LDS stack exceeds 64 KiB).
- * refill: idle lanes that make a wave claim new rays, 1..64 (0 = 24 for
- * camera rays and 16 for shadow rays): the rays a wave takes per refill. layout: 0 = traverse the compact
- * breadth-first node layout (8 bytes per node, children contiguous) whenever
- * the node array is a proper tree, 1 = always the direct 32-byte child
- * blocks. stack: 0 = per-lane traversal stacks in LDS, 1 = in global memory.
+ * refill: idle lanes that make a wave claim new rays, 1..64 (0: camera rays
+ * at 180 idle lane-steps since the last refill or 48 idle lanes, shadow rays
+ * at 16 idle lanes). layout: 0 = traverse the compact breadth-first node
+ * layout (8 bytes per node, children contiguous) whenever the node array is a
+ * proper tree, 1 = always the direct 32-byte child blocks. stack: 0 = per-lane traversal stacks in LDS, 1 = in global memory.
  * reorder: 1 = shadow rays in direction-octant order per light. graph: 1 =
  * capture the batch's launches into a hipGraph and replay it while the
  * launch configuration is unchanged. strip: order of the 8x8 pixel tiles,
@@ -245,9 +245,8 @@ int qbt_profile_end(qbt_ctx* ctx, qbt_profile* out);
  * merge: whether an exact render (no surrogate, no sample collection,
  * reorder 0) traces its camera and shadow rays in one persistent launch, the
  * shadow rays of finished pixels taken by waves whose camera work has run
- * dry, instead of a camera launch, then a shadow launch: 0 = never, 1 =
- * where it pays (default: nowhere at present), 2 = always. Results never
- * depend on these. */
+ * dry, instead of a camera launch, then a shadow launch: 0 and 1 (the
+ * default) = never, 2 = always. Results never depend on these. */
 typedef struct qbt_tuning {
     int path;
     int block_threads;
@@ -267,7 +266,7 @@ int qbt_set_tuning(qbt_ctx* ctx, const qbt_tuning* in);
  * counting/collection flags are dropped) under candidate tunings of the
  * wavefront path - coordinate descent over block_threads {64, 128, 256},
  * refill {defaults, 8, 16, 24, 32, 48}, stack {LDS, global}, reorder {0, 1}
- * and merge {0, 1, 2} (merge takes effect with reorder 0), two
+ * and merge {0, 1, 2} (0 and 1 are the same; 2 takes effect with reorder 0), two
  * sweeps, a candidate kept only if it is at least 1% faster - and leaves the
  * fastest set on the context. results (up to max_results) receive every
  * timed candidate, *nresults how many were timed. reps: timed renders per

@@ -33,9 +33,9 @@
  * HBM is the bound, half of it the scattered writes of child blocks and
  * reference map (node order is point order, record order is key order).
  * Whole calls, depth 12: 10M points (29M nodes) 3.3 ms with kept scratch and
- * 3.7 without, against 6.1 and 13.6 with a reduction by key, a scan and four
- * scatter passes per depth; 2M points (8M nodes) 0.90 against 2.0; 90M
- * points (157M nodes) 22.7 against 51. Scratch is 24 bytes a point (20 up to
+ * 3.8 without, against 6.1 and 13.4 with a reduction by key, a scan and four
+ * scatter passes per depth; 2M points (8M nodes) 0.89 against 2.0; 90M
+ * points (158M nodes) 22.7 against 51. Scratch is 24 bytes a point (20 up to
  * 10 levels).
  */
 #include <hip/hip_runtime.h>

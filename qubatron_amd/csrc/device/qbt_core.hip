@@ -384,7 +384,8 @@ __device__ __forceinline__ unsigned trace_batch(const SceneDev& s, uint32_t n, G
 
 /* Batched octree_trace_line (SEM: kSemShader, kSemCpu or kSemParticle). 200k
  * rays (0.5 a lane) of the 10M-point scene: 523 us with one thread per ray
- * and every wave waiting for its longest, 233 us as work items. */
+ * and every wave waiting for its longest, 233 us as work items (183 with the
+ * present step). */
 template <bool CMP, bool DUAL, int SEM, bool GRID>
 __global__ void __launch_bounds__(256) k_trace_rays(SceneDev s, const float* __restrict__ org,
                                                      const float* __restrict__ dir, uint32_t n, GridRule rule,

@@ -186,7 +186,7 @@ struct qbt_ctx {
     uint64_t     aborted         = 0;
     int          iter_cap        = 1 << 22;
     int          tune_block      = 0;
-    int          tune_refill     = 0;  /* idle lanes that trigger a wave refill (1..64; 0 = 24 camera, 16 shadow) */
+    int          tune_refill     = 0;  /* idle lanes that trigger a wave refill (1..64; 0: camera rays by idle lane-steps (refill_rule), others 16) */
     int          path            = 1;  /* 0 = fused per-pixel kernel, 1 = wavefront stages */
     int          num_cus         = 256;
     /* wavefront render buffers */
@@ -206,7 +206,7 @@ struct qbt_ctx {
     int          tune_reorder = 0; /* shadow rays in direction-octant order (measured: no gain) */
     int          tune_graph   = 1; /* replay batched renders from a captured hipGraph */
     int          tune_strip   = 0; /* tile order: 0 row-major, S > 0 vertical strips of S tiles */
-    int          tune_merge   = 1; /* exact renders: camera and shadow rays in one launch (k_frame): 2 always; 0 and 1 never (1: where it pays, nowhere at present) */
+    int          tune_merge   = 1; /* exact renders: camera and shadow rays in one launch (k_frame): 2 always; 0 and 1 never */
     /* captured render graph and the launch configuration it was captured for */
     hipGraph_t           graph      = nullptr;
     hipGraphExec_t       graph_exec = nullptr;

@@ -1158,10 +1158,11 @@ static int render_batch_t(qbt_ctx* c, const SceneDev& s, const BatchHost& bh, co
     /* Tuning merge 2: camera and shadow rays of an exact render in one launch
      * (k_frame). It was the faster form of some renders while the end of the
      * camera launch left the SIMDs to a few long rays; with those rays shared
-     * out (drain) it is not: 90M points, 1920x1080, 2 lights, three views
-     * 2.22 + 4.09 + 3.46 ms against 2.14 + 4.12 + 3.39 for the two launches,
-     * and 12 views with 4 lights of a scene where a fifth of the pixels are
-     * shaded 4.9 against 3.3 ms (a hand-over slot for every pixel and light). */
+     * out (drain) it is not: calls over 90M points, 1920x1080, 2 lights, three
+     * views 1.89, 3.35 and 2.83 ms against 1.70, 3.24 and 2.66 for the two
+     * launches, and 12 views with 4 lights of 10M points, two sets, 4.6 and
+     * 4.2 against 3.0 and 2.6 ms (a hand-over slot for every pixel and light).
+     * Tuning 0 and 1 are the two launches. */
     const bool merged = c->tune_merge == 2 && nl > 0 && !surrogate && !collect && !reorder;
     if (merged && (rc = c->dev_alloc(c->wb_slots, (size_t) nitems * 16 * nl))) return rc;
     /* shadow items are at most one per batch pixel and light */

@@ -24,14 +24,15 @@
  * the same operations). Rays keep their lane's identity: the owner's outputs
  * are written by the owner.
  *
- * What bounds it: the latency of a step (about 1 us for a wave alone on its
- * SIMD: 400 instructions and a dependent gather), times the steps of the
- * longest segment. A round costs a few dozen instructions and LDS exchanges,
- * so kBurst trades their number against the time a lane idles. Measured, the
- * shadow launch of the 10M-point scene at 1920x1080 (0.55M rays, the longest
- * 375 steps): 632 us without sharing, 407, 408, 444 with bursts of 4, 8 and
- * 16 steps; k_shadow of a 320x240 frame (28k rays): 204, then 91, 95, 126;
- * its k_primary (77k rays): 175, then 141, 128, 136.
+ * What bounds it: the latency of a step (about 0.9 us for a wave alone on its
+ * SIMD: some 200 vector instructions and a dependent gather), times the steps
+ * of the longest segment. A round costs a few dozen instructions and LDS
+ * exchanges, so kBurst trades their number against the time a lane idles.
+ * Measured with bursts of 4, 8 and 16 steps: k_primary + k_shadow of 320x240
+ * frames of 1M points (three poses) 209, 197, 224 us, 191, 187, 188 and 104,
+ * 107, 122; k_shadow of 1920x1080 frames of 10M points 357, 355, 371 us, 465,
+ * 464, 482 and 112, 111, 111. Without sharing (with an earlier, longer step)
+ * a shadow launch of the latter kind took 632 us against 408.
  *
  * Every step of the loop takes a segment further or ends it, no lane waits
  * for another inside a burst, and the loop ends when no ray is left.
